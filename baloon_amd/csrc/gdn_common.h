@@ -188,6 +188,35 @@ __device__ __forceinline__ void q81_store(float v, int lane, uint8_t* blk) {
     }
 }
 
+// q81_store for a lane that holds 4 consecutive values, entries 4 (lane & 7) .. + 3 of the block of
+// its 8 lanes: the same bytes (the butterfly's steps 16, 8, 4 cross lanes, 2 and 1 stay inside).
+// All 64 lanes call it; blk == nullptr stores nothing.
+__device__ __forceinline__ void q81_store4(const v4f& v, int lane, uint8_t* blk) {
+    float m = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    v4f s = v;
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) {
+        m = fmaxf(m, __shfl_xor(m, off, kWave));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = s[e] + __shfl_xor(s[e], off, kWave);
+    }
+    const float sum = (s[0] + s[2]) + (s[1] + s[3]);
+    const float d = fminf(m / 127.0f, kHalfMax);
+    uint32_t q = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int c = d == 0.0f ? 0 : (int)fminf(fmaxf(roundf(v[e] / d), -127.0f), 127.0f);
+        q |= (uint32_t)(uint8_t)(int8_t)c << (8 * e);
+    }
+    if (!blk) return;
+    *reinterpret_cast<uint32_t*>(blk + 4 + 4 * (lane & 7)) = q;
+    if ((lane & 7) == 0) {
+        const float sc = fminf(fmaxf(sum, -kHalfMax), kHalfMax);
+        const uint32_t hd = __builtin_bit_cast(uint16_t, (_Float16)d), hs = __builtin_bit_cast(uint16_t, (_Float16)sc);
+        *reinterpret_cast<uint32_t*>(blk) = hd | (hs << 16);
+    }
+}
+
 // Sum of v^2 over the wave, the same bits in every lane and in every kernel that calls it:
 // each square is rounded before the sums (left to itself the compiler fuses it into the
 // first DPP add, whose result then differs between lanes), and lane 0's total is broadcast.
@@ -236,6 +265,26 @@ __device__ __forceinline__ void out_gate_head(const OutGate& g, size_t row, floa
 }
 __device__ __forceinline__ void out_gate_head(const OutGate& g, size_t row, float lo, float hi, int lane) {
     out_gate_head(g, row, lo, hi, lane, gate_in(g, row, lane));
+}
+
+// The same norm of a row held by a half wave, lane l its columns 4 (l & 31) .. + 3: the lane's four
+// results from its outputs, weights and gate inputs. The sum of squares is again (columns 0..63) +
+// (columns 64..127). All 64 lanes call it; the same arguments give the same bits wherever it is
+// inlined (nothing is left for the compiler to contract).
+__device__ __forceinline__ v4f gate_row4(const OutGate& g, const v4f& o, const v4f& nrm, const uint2& z) {
+    float sq = fmaf(o[0], o[0], fmaf(o[1], o[1], fmaf(o[2], o[2], o[3] * o[3])));
+    __asm__("" : "+v"(sq));                                  // no part of it fused into the sums
+    const float inv = rsqrtf(fmaf(pair_sum16(row_sum16(sq)), 1.0f / kD, g.eps));
+    const float zf[4] = {__uint_as_float(z.x << 16), __uint_as_float(z.x & 0xffff0000u), __uint_as_float(z.y << 16),
+                         __uint_as_float(z.y & 0xffff0000u)};
+    v4f y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float v = o[e] * inv * nrm[e] * sigmoid_fast(zf[e]);
+        __asm__("" : "+v"(v));                               // nor this product into a caller's sum
+        y[e] = v;
+    }
+    return y;
 }
 
 // ---------------------------------------------------------------------------------------

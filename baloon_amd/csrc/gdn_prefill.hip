@@ -21,8 +21,10 @@
 // Kernels, in stream order, per window of chunks (the workspace holds one window's chunk
 // operands; windows run one after the other, with identical results for any window size):
 //   plan_kernel    (once, n_seq > 1 only) clamps cu_seqlens to a non-decreasing sequence in
-//                  [0, total_T], builds the chunk table and lists the non-empty sequences;
-//                  a single sequence's geometry comes from cu[0], cu[1] directly
+//                  [0, total_T], decides for batches of many sequences which of them run one
+//                  workgroup per sequence and heads (seq_kernel, gdn_prefill_seq.hip) and builds the
+//                  chunk table of the others; a single sequence's geometry comes from cu[0], cu[1]
+//                  directly
 //   tri_kernel     per (chunk, q/k head): conv and L2 norms of the chunk's q and k rows, the
 //                  K K^T and Q K^T lower block triangles once for all the v heads mapped to the
 //                  q/k head, then per v head the decay scan and beta, A and M, T = (I + A)^-1
@@ -37,103 +39,12 @@
 // Every dense product runs on split-bf16 MFMA (three bf16 products per fp32 product, ~2^-16
 // relative error); only the 16 x 16 diagonal blocks of T are inverted in fp32 arithmetic.
 // The chunked result stays within ~1e-5 (state) of the token-by-token recurrence in double.
-#include "gdn_common.h"
+#include "gdn_prefill_seq.h"
 
 namespace ixg {
 namespace {
 
-constexpr int kChunk = 64;
 constexpr int kPlanThreads = 1024;
-
-// ---------------------------------------------------------------------------------------
-// Workspace layout (host and device agree through this struct)
-// ---------------------------------------------------------------------------------------
-// The chunk tables cover every chunk; the chunk operands cover one window of W chunks (the
-// kernels run window by window, W chosen to fit the caller's workspace).
-struct Ws {
-    int32_t* seq_lo;     // [n_seq + 1] clamped token offsets
-    int32_t* chunk_off;  // [n_seq + 1] first chunk of each sequence; chunk_off[n_seq] = #chunks
-    int4* chunk_rec;     // [NC] {sequence, first token, sequence start, sequence end}
-    uint8_t* Tf;         // [W][h_v] T' = (I + A)^-1 diag(beta) (64 x 64) as split-bf16 A fragments
-                         // (the nonzero ones, kTriFragBytes per head)
-    uint8_t* Mf;         // [W][h_v] M (64 x 64) as split-bf16 A fragments (kFragMBytes per head)
-    float* G;            // [W][h_v][2][64] decay factors exp(G_last - G_t), then exp(G_t), of the
-                         // inclusive cumulative log decay G (padded rows repeat the last)
-    uint8_t* Kp;         // [W][h_k] normalised keys as split-bf16 planes in the chain's LDS layout
-    uint16_t* Qf;        // [W][h_k] Q (64 x 128) as split-bf16 A fragments
-};
-constexpr int kWsSections = 8;
-constexpr int kTriFragBytes = 10 * 1024;                // T' of one (chunk, v head)
-constexpr int kFragMBytes = 16 * 1024;                  // M of one (chunk, v head)
-constexpr int kPRow = 2 * 128;                          // key plane row: 128 bf16 as 16 chunks of 16 bytes
-constexpr int kKPlane = 64 * kPRow;                     // one plane (hi or lo) of 64 keys
-constexpr int kKSlot = 2 * kKPlane;                     // hi, then lo: 32 KiB
-// Chunk j of key row t is stored at chunk j ^ kswz(t) of its row: the two 2-bit halves of
-// t mod 16 swapped, so that the chain's 16-byte fragment reads (16 rows, one chunk column) and
-// its transposing 8-byte reads (4 rows x 4 chunk columns per lane group) hit 16 distinct chunks.
-__host__ __device__ constexpr int kswz(int t) { return ((t & 3) << 2) | ((t >> 2) & 3); }
-
-inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-
-// Chunks of (n_seq, T) at most: each sequence adds at most one partial chunk.
-inline size_t max_chunks(int n_seq, int T) { return (size_t)(T + kChunk - 1) / kChunk + (size_t)n_seq; }
-
-// Byte offsets of every workspace section for (n_seq, T) in windows of W chunks; returns the
-// total size.
-inline size_t ws_layout(const ix_gdn_cfg* c, int n_seq, int T, size_t W, size_t off[kWsSections]) {
-    const size_t NC = max_chunks(n_seq, T);
-    const size_t sz[kWsSections] = {
-        sizeof(int32_t) * (n_seq + 1), sizeof(int32_t) * (n_seq + 1), sizeof(int4) * NC,
-        (size_t)kTriFragBytes * W * c->h_v, (size_t)kFragMBytes * W * c->h_v, sizeof(float) * W * c->h_v * 2 * kChunk, (size_t)kKSlot * W * c->h_k,
-        sizeof(uint16_t) * W * c->h_k * 4 * 4 * 2 * 512,
-    };
-    size_t pos = 0;
-    for (int i = 0; i < kWsSections; ++i) { off[i] = pos; pos += align256(sz[i]); }
-    return pos;
-}
-
-inline Ws ws_bind(char* base, const size_t off[kWsSections]) {
-    Ws w;
-    w.seq_lo = reinterpret_cast<int32_t*>(base + off[0]);
-    w.chunk_off = reinterpret_cast<int32_t*>(base + off[1]);
-    w.chunk_rec = reinterpret_cast<int4*>(base + off[2]);
-    w.Tf = reinterpret_cast<uint8_t*>(base + off[3]);
-    w.Mf = reinterpret_cast<uint8_t*>(base + off[4]);
-    w.G = reinterpret_cast<float*>(base + off[5]);
-    w.Kp = reinterpret_cast<uint8_t*>(base + off[6]);
-    w.Qf = reinterpret_cast<uint16_t*>(base + off[7]);
-    return w;
-}
-
-struct PrefillParams {
-    Layer L;
-    Ws ws;
-    const int32_t* cu;          // [n_seq + 1]
-    const uint16_t* x;          // [T][C]
-    uint16_t* conv_state;       // [n_seq][C][dc-1]
-    const uint16_t* a;          // [T][h_v]
-    const uint16_t* b;          // [T][h_v]
-    float* state;               // [n_seq][h_v][d_v][d_k]
-    float* o;                   // [T][h_v][128], the window's rows (o_win), or null
-    uint16_t* o_bf16;           // [T][h_v][128] or null
-    int n_seq, T, NC;
-    int single;                 // n_seq == 1: no plan pass; the geometry comes from cu[0], cu[1]
-    int cb, W;                  // the window: chunks cb .. cb + W - 1
-    int G;                      // chain workgroups per (v head, strip) in a window (1 for n_seq == 1)
-    int o_win;                  // o holds the window's tokens only (row 0 = its first token)
-};
-
-// Clamped bounds [lo, hi) of sequence s: the plan's seq_lo (running maximum of the offsets,
-// clamped to [0, T]), or for a single sequence the same two values from cu directly.
-__device__ __forceinline__ void seq_bounds(const PrefillParams& p, int s, int& lo, int& hi) {
-    if (p.single) {
-        lo = min(max(p.cu[0], 0), p.T);
-        hi = max(min(max(p.cu[1], 0), p.T), lo);
-    } else {
-        lo = p.ws.seq_lo[s];
-        hi = p.ws.seq_lo[s + 1];
-    }
-}
 
 // ---------------------------------------------------------------------------------------
 // plan: one workgroup of 1024 threads, block scans in tiles of 1024 sequences
@@ -167,7 +78,10 @@ __device__ int block_inclusive_scan(int v, int* wave_tot) {
 __global__ void __launch_bounds__(kPlanThreads) plan_kernel(const PrefillParams p) {
     __shared__ int wave_tot[kPlanThreads / kWave];
     __shared__ int carry;
+    __shared__ int hist[kPlanThreads];
+    __shared__ unsigned long long best[kPlanThreads / kWave];
     const int tid = threadIdx.x, n = p.n_seq;
+    auto chunks_of = [&](int s) { return (p.ws.seq_lo[s + 1] - p.ws.seq_lo[s] + kChunk - 1) / kChunk; };
     // seq_lo[s] = clamp(max(cu[0..s]), 0, T), s = 0..n
     int run = 0;                                                       // carry, same in every thread
     for (int base = 0; base <= n; base += kPlanThreads) {
@@ -180,11 +94,54 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(const PrefillParams 
         run = carry;
         __syncthreads();
     }
-    // chunk_off = exclusive prefix sum of ceil(len / 64)
+    // With by_seq, the sequences of more than `longest` chunks go through the chunk table and the
+    // others, listed longest first, to seq_kernel; `longest` minimises the two parts' time. Thread v
+    // prices v: seq_kernel runs its longest sequence's chunks one after the other (cost_seq each)
+    // or, if that is more, the GPU's share of all its work (cost_work per chunk); the windows take
+    // cost_win per chunk of the table.
+    int longest = 0;
+    if (p.by_seq) {
+        hist[tid] = 0;
+        __syncthreads();
+        for (int s = tid; s < n; s += kPlanThreads) {
+            const int c = chunks_of(s);
+            atomicAdd(&hist[min(c, kPlanThreads - 1)], c);
+        }
+        __syncthreads();
+        const int upto = block_inclusive_scan<false>(hist[tid], wave_tot);   // chunks of lengths <= tid
+        if (tid == kPlanThreads - 1) carry = upto;
+        __syncthreads();
+        const float cost = p.cost_win * (float)(carry - upto) + fmaxf(p.cost_seq * (float)tid, p.cost_work * (float)upto);
+        // the least cost, the shortest length on a tie: (cost, length) as one 64-bit key
+        unsigned long long key = ((unsigned long long)__float_as_uint(cost) << 32) | (unsigned)tid;
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+            const unsigned long long o = __shfl_xor(key, off, kWave);
+            key = o < key ? o : key;
+        }
+        if ((tid & (kWave - 1)) == 0) best[tid / kWave] = key;
+        __syncthreads();
+        key = best[0];
+        for (int i = 1; i < kPlanThreads / kWave; ++i) key = best[i] < key ? best[i] : key;
+        longest = (int)(key & 0xffffffffu);
+        if (longest == kPlanThreads - 1) longest = INT_MAX;
+        __syncthreads();
+        hist[tid] = 0;                                                 // counting sort, longest first
+        __syncthreads();
+        for (int s = tid; s < n; s += kPlanThreads) atomicAdd(&hist[kPlanThreads - 1 - min(chunks_of(s), kPlanThreads - 1)], 1);
+        __syncthreads();
+        const int v = hist[tid], first = block_inclusive_scan<false>(v, wave_tot) - v;
+        hist[tid] = first;
+        __syncthreads();
+        for (int s = tid; s < n; s += kPlanThreads)
+            p.ws.order[atomicAdd(&hist[kPlanThreads - 1 - min(chunks_of(s), kPlanThreads - 1)], 1)] = s;
+    }
+    auto tabled = [&](int cnt) { return p.by_seq && cnt <= longest ? 0 : cnt; };
+    // chunk_off = exclusive prefix sum of ceil(len / 64), of the sequences in the table
     run = 0;
-    for (int base = 0; base <= n; base += kPlanThreads) {
+    for (int base = 0; base < n + 1; base += kPlanThreads) {
         const int s = base + tid;
-        const int cnt = s < n ? (p.ws.seq_lo[s + 1] - p.ws.seq_lo[s] + kChunk - 1) / kChunk : 0;
+        const int cnt = s < n ? tabled(chunks_of(s)) : 0;
         const int inc = block_inclusive_scan<false>(cnt, wave_tot) + run;
         if (s <= n) p.ws.chunk_off[s] = inc - cnt;
         if (tid == kPlanThreads - 1) carry = inc;
@@ -208,7 +165,6 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(const PrefillParams 
 // Chunk geometry: sequence, first token, tokens in the chunk, position of the first token
 // within its sequence. Returns false for grid slots beyond the chunk count.
 // One load for the whole geometry (the chunk count is read alongside, independently).
-struct ChunkGeo { int s, t0, len, pos0, lo; };
 __device__ __forceinline__ bool chunk_geo(const PrefillParams& p, int c, ChunkGeo& g) {
     if (p.single) {                                   // chunk c of the only sequence
         int lo, hi;
@@ -231,141 +187,6 @@ __device__ __forceinline__ bool chunk_geo(const PrefillParams& p, int c, ChunkGe
     g.len = min(kChunk, r.w - g.t0);
     g.pos0 = g.t0 - g.lo;
     return true;
-}
-
-// Tokens [t0, t1) of the window's chunks (consecutive chunks cover consecutive tokens); t0 = t1
-// for a window past the last chunk.
-__device__ __forceinline__ void window_tokens(const PrefillParams& p, int& t0, int& t1) {
-    ChunkGeo a, b;
-    t0 = t1 = 0;
-    if (!chunk_geo(p, p.cb, a)) return;
-    int nc;
-    if (p.single) {
-        int lo, hi;
-        seq_bounds(p, 0, lo, hi);
-        nc = (hi - lo + kChunk - 1) / kChunk;
-    } else {
-        nc = p.ws.chunk_off[p.n_seq];
-    }
-    chunk_geo(p, min(p.cb + p.W, nc) - 1, b);               // chunk cb exists, so this one does
-    t0 = a.t0;
-    t1 = b.t0 + b.len;
-}
-
-// ---------------------------------------------------------------------------------------
-// Conv of 16 consecutive tokens of a chunk for the channel pair (ch, ch + 1), one pair per
-// lane, so that every x access of a wave is one 256-byte row segment. Tokens tb .. tb + n - 1
-// of the chunk (n wave-uniform, 1..16); the history of the first one comes from x or, before
-// the sequence start, from the sequence's conv state ([C][dc-1] per sequence: channel ch's
-// entries, then channel ch+1's).
-// The loads and the arithmetic are separate steps, so that a wave can issue the loads well
-// before it needs the rows (and before stores it issues in between, which its later waits
-// would otherwise include).
-// ---------------------------------------------------------------------------------------
-constexpr int kConvTok = 16;
-
-// The loads are unconditional and nothing touches the loaded words before conv_run: a
-// load on one path only, or any use of a loaded value, makes the wave wait for every load
-// it has in flight. Every row index is clamped into the chunk's tokens, so a wave whose
-// rows all lie past the chunk end (n = 0) reads valid rows, whose results are discarded.
-template <int DC>
-struct ConvIn {
-    uint32_t h0[DC - 1], h1[DC - 1];    // history of the first token (one bf16 each), oldest first
-    uint32_t xs[kConvTok];              // bf16 pairs: inputs of the tokens (rows past n repeat row n-1)
-    uint32_t w[DC];                     // bf16 pairs: conv weights of channel ch, then ch + 1
-};
-
-template <int DC>
-__device__ __forceinline__ void conv_load(const PrefillParams& p, const ChunkGeo& g, int lo, int ch, int tb, int n,
-                                          ConvIn<DC>& in) {
-    const Layer& L = p.L;
-#pragma unroll
-    for (int i = 0; i < DC - 1; ++i) {
-        const int pos = min(g.pos0 + tb - (DC - 1) + i, g.pos0 + g.len - 1);   // wave-uniform
-        const uint16_t* xp = p.x + (size_t)(lo + max(pos, 0)) * L.C + ch;
-        const uint16_t* sp = p.conv_state + ((size_t)g.s * L.C + ch) * (DC - 1) + (DC - 1) + min(pos, -1);
-        in.h0[i] = *(pos >= 0 ? xp : sp);
-        in.h1[i] = *(pos >= 0 ? xp + 1 : sp + (DC - 1));
-    }
-#pragma unroll
-    for (int t = 0; t < kConvTok; ++t)
-        in.xs[t] = *reinterpret_cast<const uint32_t*>(p.x + (size_t)(g.t0 + min(tb + min(t, n - 1), g.len - 1)) * L.C + ch);
-    // conv_w is [C][dc]: the two channels' 2 dc weights are dc aligned words (ch is even)
-    const uint32_t* wp = reinterpret_cast<const uint32_t*>(L.conv_w + (size_t)ch * DC);
-#pragma unroll
-    for (int i = 0; i < DC; ++i) in.w[i] = wp[i];
-}
-
-__device__ __forceinline__ float bf16_half(uint32_t word, int half) {
-    return __uint_as_float(half ? (word & 0xffff0000u) : (word << 16));
-}
-
-template <int DC, bool SILU>
-__device__ __forceinline__ void conv_run(ConvIn<DC> in, float (&y0)[kConvTok], float (&y1)[kConvTok]) {
-    // Pin the words here: the compiler would otherwise hoist their unpacking up to the loads,
-    // which then wait for the data right after issue.
-#pragma unroll
-    for (int i = 0; i < DC - 1; ++i) { __asm__ volatile("" : "+v"(in.h0[i])); __asm__ volatile("" : "+v"(in.h1[i])); }
-#pragma unroll
-    for (int t = 0; t < kConvTok; ++t) __asm__ volatile("" : "+v"(in.xs[t]));
-#pragma unroll
-    for (int i = 0; i < DC; ++i) __asm__ volatile("" : "+v"(in.w[i]));
-    float h0[DC - 1], h1[DC - 1], w0[DC], w1[DC];
-#pragma unroll
-    for (int i = 0; i < DC - 1; ++i) { h0[i] = __uint_as_float(in.h0[i] << 16); h1[i] = __uint_as_float(in.h1[i] << 16); }
-#pragma unroll
-    for (int i = 0; i < DC; ++i) {
-        w0[i] = bf16_half(in.w[i >> 1], i & 1);
-        w1[i] = bf16_half(in.w[(DC + i) >> 1], (DC + i) & 1);
-    }
-#pragma unroll
-    for (int t = 0; t < kConvTok; ++t) {
-        const float x0 = bf16_half(in.xs[t], 0), x1 = bf16_half(in.xs[t], 1);
-        float a0 = 0.0f, a1 = 0.0f;
-#pragma unroll
-        for (int i = 0; i < DC - 1; ++i) { a0 = fmaf(h0[i], w0[i], a0); a1 = fmaf(h1[i], w1[i], a1); }
-        a0 = fmaf(x0, w0[DC - 1], a0);
-        a1 = fmaf(x1, w1[DC - 1], a1);
-        if constexpr (SILU) { a0 = a0 * sigmoid_f(a0); a1 = a1 * sigmoid_f(a1); }
-        y0[t] = a0;
-        y1[t] = a1;
-#pragma unroll
-        for (int i = 0; i < DC - 2; ++i) { h0[i] = h0[i + 1]; h1[i] = h1[i + 1]; }
-        h0[DC - 2] = x0;
-        h1[DC - 2] = x1;
-    }
-}
-
-// ---------------------------------------------------------------------------------------
-// commit: the rolling conv history of channel ch after sequence s, tokens lo .. lo+len-1
-// (len > 0); run by the chain kernel after every read of the old history
-// ---------------------------------------------------------------------------------------
-// The new history's dc-1 values, loaded (hist_fetch), then stored (hist_put) once they have
-// arrived, so that a wave can issue other loads in between.
-struct HistNew { uint16_t v[3]; };
-__device__ __forceinline__ HistNew hist_fetch(const PrefillParams& p, int ch, int lo, int len, int s) {
-    const Layer& L = p.L;
-    const uint16_t* st = p.conv_state + ((size_t)s * L.C + ch) * (L.dc - 1);
-    // extended history [old (dc-1 values) | the sequence's inputs]; the new history is its
-    // last dc-1 entries, i.e. entries len .. len+dc-2. An entry below dc-1 is old history.
-    const uint16_t o0 = st[0], o1 = L.dc > 2 ? st[1] : (uint16_t)0, o2 = L.dc > 3 ? st[2] : (uint16_t)0;
-    // Entries j >= dc-1 are not stored; their token index is clamped into the sequence, so
-    // that no load reaches past its last token.
-    HistNew h;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const int ext = len + j;                               // index into the extended history
-        const int pos = ext - (L.dc - 1);                      // token position when >= 0
-        h.v[j] = pos >= 0 ? p.x[(size_t)(lo + min(pos, len - 1)) * L.C + ch] : (ext == 0 ? o0 : ext == 1 ? o1 : o2);
-    }
-    return h;
-}
-__device__ __forceinline__ void hist_put(const PrefillParams& p, int ch, int s, const HistNew& h) {
-    const Layer& L = p.L;
-    uint16_t* st = p.conv_state + ((size_t)s * L.C + ch) * (L.dc - 1);
-    st[0] = h.v[0];
-    if (L.dc > 2) st[1] = h.v[1];
-    if (L.dc > 3) st[2] = h.v[2];
 }
 
 // ---------------------------------------------------------------------------------------
@@ -392,15 +213,6 @@ __device__ __forceinline__ void store_frag(uint8_t* base, int m, int ks, int nks
     *reinterpret_cast<bf8*>(base + 2 * frag_at(m, ks, nks, 1, lane)) = lo;
 }
 
-// T' (64 x 64, lower triangular, split) stores its 6 nonzero fragments back to back, (0, 0),
-// (1, 0), (2, 0), (2, 1), (3, 0), (3, 1); (0, 0) and (2, 1) pair a diagonal block with a zero
-// block, so only entries 0..3 of each lane are stored (8 bytes a lane, 512 a plane). Byte offset
-// of a lane's part of one plane:
-__host__ __device__ constexpr bool tri_half(int m, int ks) { return (m == 0 && ks == 0) || (m == 2 && ks == 1); }
-__device__ __forceinline__ int tri_frag_at(int m, int ks, int plane, int lane) {
-    const int off = m == 0 ? 0 : m == 1 ? 1024 : m == 2 ? (ks ? 5120 : 3072) : (ks ? 8192 : 6144);
-    return off + (tri_half(m, ks) ? plane * 512 + lane * 8 : plane * 1024 + lane * 16);
-}
 __device__ __forceinline__ void store_tri_frag(uint8_t* base, int m, int ks, int lane, const bf8& hi, const bf8& lo) {
     if (tri_half(m, ks)) {
         const u4x h = __builtin_bit_cast(u4x, hi), l = __builtin_bit_cast(u4x, lo);
@@ -438,14 +250,6 @@ constexpr int kQKPlane = kChunk * 256;                   // bytes per plane
 __device__ __forceinline__ int qk_off(int t, int ch) {
     return t * 256 + ((((ch >> 3) ^ (t & 15))) << 4) + ((ch & 7) << 1);
 }
-typedef __attribute__((address_space(3))) uint8_t lds_u8;
-typedef short v4s __attribute__((ext_vector_type(4)));
-// Transposing 8-byte LDS read of 16-bit elements (gfx950 ds_read_b64_tr_b16).
-__device__ __forceinline__ uint2 lds_tr16(const lds_u8* a) {
-    typedef __attribute__((address_space(3))) v4s lds_v4s;
-    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)a));
-}
-
 // The 10 blocks (br, bc) of the 4 x 4 lower block triangle, 16 x 16 each: wave w takes
 // i = w, w+4, w+8. The order gives each wave whole 32-column halves of block rows: wave 0
 // (1,0) (1,1) (0,0), wave 1 (2,0) (2,1) (2,2), wave 2 (3,0) (3,1), wave 3 (3,2) (3,3), so
@@ -456,23 +260,6 @@ __device__ __forceinline__ void tri_block(int i, int& br, int& bc) {
     bc = (0x8d580 >> (2 * i)) & 3;                      // 0 0 0 2 1 1 1 3 0 2
 }
 
-// 16x16x16 bf16 MFMA operands: A lane l holds A[l%16][4 (l/16) + e], B lane l holds
-// B[4 (l/16) + e][l%16], e = 0..3, and the accumulator's lane l holds C[4 (l/16) + r][l%16],
-// so an accumulator split to bf16 is the next product's B operand as it stands.
-typedef short bf4 __attribute__((ext_vector_type(4)));
-struct Split4 { bf4 h, l; };
-__device__ __forceinline__ Split4 split4(const v4& x) {
-    uint32_t h0, l0, h1, l1;
-    split2(x[0], x[1], h0, l0);
-    split2(x[2], x[3], h1, l1);
-    return Split4{__builtin_bit_cast(bf4, uint2{h0, h1}), __builtin_bit_cast(bf4, uint2{l0, l1})};
-}
-// c += A B on split operands (hi hi + hi lo + lo hi).
-__device__ __forceinline__ v4 mfma16_split(const Split4& a, const Split4& b, v4 c) {
-    c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.h, b.h, c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.h, b.l, c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a.l, b.h, c, 0, 0, 0);
-}
 // A operand of the 16 x 16 block at (r0, c0) of an LDS matrix with row stride kTS, times s.
 __device__ __forceinline__ Split4 block_a(const float* m, int r0, int c0, int lane, float s) {
     return split4(s * *reinterpret_cast<const v4*>(m + (r0 + (lane & 15)) * kTS + c0 + 4 * (lane >> 4)));
@@ -870,9 +657,6 @@ constexpr int kChainLds = kOffV1 + 4 * kPlane;          // 135,952 bytes
 // V of chunk c_k (4 row tiles, accumulator layout): written in alpha_{k-1}, read in alpha_k.
 __device__ __forceinline__ int v_buf(int k) { return (k & 1) ? kOffV1 : kOffV; }
 
-typedef __attribute__((address_space(3))) bf8 lds_bf8;
-typedef __attribute__((address_space(3))) v4 lds_v4;
-
 // This lane's address in an LDS area at byte offset off (which includes the lane's own part),
 // made opaque to the compiler: reads and writes at base + (a constant below 64 KiB) then use
 // the instruction's immediate offset, where the folded address of an area above 64 KiB
@@ -881,53 +665,6 @@ __device__ __forceinline__ lds_u8* lane_at(uint8_t* lds, int off) {
     lds_u8* b = (lds_u8*)lds + off;
     __asm__ volatile("" : "+v"(b));
     return b;
-}
-
-// B operand of one 32-wide k-step from two stacked accumulator tiles (kperm order), split.
-__device__ __forceinline__ void split_tiles(const v4& a, const v4& b, bf8& hi, bf8& lo) {
-    uint32_t h0, h1, h2, h3, l0, l1, l2, l3;
-    split2(a[0], a[1], h0, l0);
-    split2(a[2], a[3], h1, l1);
-    split2(b[0], b[1], h2, l2);
-    split2(b[2], b[3], h3, l3);
-    hi = __builtin_bit_cast(bf8, u4x{h0, h1, h2, h3});
-    lo = __builtin_bit_cast(bf8, u4x{l0, l1, l2, l3});
-}
-
-// Key slots hold each 32-channel block of a key row in kperm order: channels 4 a .. 4 a + 3,
-// then 16 + 4 a .. 16 + 4 a + 3, for a = 0..3, i.e. channel 32 b + 16 h + 4 a + e sits at
-// position 32 b + 8 a + 4 h + e.
-// K fragment (token tile mt, channel k-step ks) of a key slot: A operand of K S. Lane
-// (li, lg4) reads row 16 mt + li, channels 32 ks + 4 lg4 .. +3 and 32 ks + 16 + 4 lg4 .. +3:
-// the 16 bytes of chunk 4 ks + lg4, stored at chunk (4 ks + lg4) ^ kswz(li) of the row.
-__device__ __forceinline__ int k_lane(int li, int lg4, int ks) {
-    return li * kPRow + 16 * ((4 * ks + lg4) ^ kswz(li));
-}
-// kb: the slot plus k_lane(li, lg4, ks).
-__device__ __forceinline__ void k_frag(const lds_u8* kb, int mt, bf8& hi, bf8& lo) {
-    const int o = mt * 16 * kPRow;
-    hi = *(const lds_bf8*)(kb + o);
-    lo = *(const lds_bf8*)(kb + kKPlane + o);
-}
-
-// K^T fragment (channel tile m, token k-step ks) of a key slot: A operand of K^T Dg, by
-// transposing reads (ds_read_b64_tr_b16: within each 16-lane group, lane j receives element
-// j & 3 of the 8-byte reads of lanes (j >> 2) + 4 e, e = 0..3). Lane i of lane group g reads
-// channels 16 m + 4 (i & 3) .. +3 of token t = 32 ks + 4 g + (i >> 2) (then of the token 16
-// later), so it receives channel 16 m + i at tokens 32 ks + 4 g + e (+ 16): entries e (4 + e)
-// of its kperm fragment chunk. Those 4 channels are half m & 1 of chunk 4 (m / 2) + (i & 3),
-// stored at chunk (4 (m / 2) + (i & 3)) ^ kswz(t) of the row (kswz(t) depends on i and g only).
-__device__ __forceinline__ int kt_lane(int i, int g, int mh) {
-    const int t = 4 * g + (i >> 2);
-    return t * kPRow + 16 * ((4 * mh + (i & 3)) ^ kswz(t));
-}
-// tb: the slot plus kt_lane(i, g, m / 2); half = m & 1.
-__device__ __forceinline__ void kt_frag(const lds_u8* tb, int half, int ks, bf8& hi, bf8& lo) {
-    const int o = ks * 32 * kPRow + half * 8;
-    const uint2 a = lds_tr16(tb + o), b = lds_tr16(tb + o + 16 * kPRow);
-    const uint2 c = lds_tr16(tb + kKPlane + o), d = lds_tr16(tb + kKPlane + o + 16 * kPRow);
-    hi = __builtin_bit_cast(bf8, u4x{a.x, a.y, b.x, b.y});
-    lo = __builtin_bit_cast(bf8, u4x{c.x, c.y, d.x, d.y});
 }
 
 // acc[j] += A_j B for four row tiles, split products; the products go tile by tile within
@@ -1363,10 +1100,6 @@ __device__ __forceinline__ void chain_output_role(const PrefillParams& p, uint8_
     const lds_u8* hbase = lane_at(lds, kOffH + lane * 16);
     const size_t row = (size_t)L.h_v * kD;
     v4 o;
-    // A window buffer for o starts at the window's first token.
-    int tw0 = 0, tw1;
-    if (p.o_win) window_tokens(p, tw0, tw1);
-    tw0 = __builtin_amdgcn_readfirstlane(tw0);              // waited for here, not in the loop
     // exp(G_t) of chunk c_k at this lane's rows, read from the value slot in alpha_k (the D wave
     // writes chunk c_{k+1}'s there in beta_k).
     const lds_u8* gmb = lane_at(lds, kOffV + 4 * kPlane + 4 * kChunk + 64 * r + 16 * lg4);
@@ -1374,7 +1107,7 @@ __device__ __forceinline__ void chain_output_role(const PrefillParams& p, uint8_
     // o rows 16 r + 4 lg4 + i of a chunk at a lane offset fixed for the run, from a chunk base
     // held in scalar registers; a full chunk stores without per-row tests.
     const uint32_t lofs = (uint32_t)((16 * r + 4 * lg4) * (int)row + li);
-    auto store = [&](const RunChunk& g) {
+    auto store = [&](const RunChunk& g, int k) {
         const int t0 = __builtin_amdgcn_readfirstlane(g.t0), len = __builtin_amdgcn_readfirstlane(g.len());
         const int tl = 16 * r + 4 * lg4;
         if (p.o_bf16) {
@@ -1389,7 +1122,8 @@ __device__ __forceinline__ void chain_output_role(const PrefillParams& p, uint8_
             }
         }
         if (p.o) {
-            float* ow = p.o + ((size_t)(t0 - tw0) * L.h_v + h) * kD + j0;
+            const int row0 = p.o_win ? (run.wk + k) * kChunk : t0;   // a window buffer has 64 rows per chunk
+            float* ow = p.o + ((size_t)row0 * L.h_v + h) * kD + j0;
             if (len >= kChunk) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) ow[lofs + (uint32_t)(i * (int)row)] = o[i];
@@ -1445,7 +1179,7 @@ __device__ __forceinline__ void chain_output_role(const PrefillParams& p, uint8_
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = a0[i] + a1[i] + a2[i];
-        store(r0);
+        store(r0, k);
         gam_k = *(const lds_v4*)gmb;                        // chunk c_{k+1}'s
         // Entries 0, 1 of row tile r of chunk c_{k+2}'s V (its x rows in xa), then chunk
         // c_{k+3}'s x rows into xb (chunk c_{k+1}'s, staged in alpha_k), and chunk c_{k+2}'s M.
@@ -1660,16 +1394,21 @@ __global__ void __launch_bounds__(256) out_gate_kernel(const float* __restrict__
     out_gate_head(g, row, o[row + lane], o[row + lane + kWave], lane);
 }
 
-// The same norm over one window's rows, for the gated prefill without a caller o: the chain
-// wrote the window's fp32 outputs to p.o, row 0 being the window's first token.
+// The same norm over one window's chunks, a wave per row in a grid of at most kGateBlocks workgroups:
+// from the window buffer (64 rows per chunk) for the gated prefill without a caller o, else from o.
+constexpr unsigned kGateBlocks = 4096;
 __global__ void __launch_bounds__(256) out_gate_window_kernel(const PrefillParams p, const OutGate g) {
-    int t0, t1;
-    window_tokens(p, t0, t1);
-    const long long r = (long long)blockIdx.x * 4 + threadIdx.x / kWave;       // row in the window
-    if (r >= (long long)(t1 - t0) * p.L.h_v) return;
     const int lane = threadIdx.x & (kWave - 1);
-    const size_t row = (size_t)r * kD;
-    out_gate_head(g, (size_t)t0 * p.L.h_v * kD + row, p.o[row + lane], p.o[row + lane + kWave], lane);
+    const long long per = (long long)kChunk * p.L.h_v, rows = per * p.W;       // h_v rows per token
+    for (long long r = (long long)blockIdx.x * 4 + threadIdx.x / kWave; r < rows; r += (long long)gridDim.x * 4) {
+        const int lc = (int)(r / per), in = (int)(r % per);
+        ChunkGeo c;
+        if (!chunk_geo(p, p.cb + lc, c)) return;
+        if (in >= c.len * p.L.h_v) continue;
+        const size_t row = ((size_t)c.t0 * p.L.h_v + in) * kD;
+        const float* o = p.o + (p.o_win ? (size_t)r * kD : row);
+        out_gate_head(g, row, o[lane], o[lane + kWave], lane);
+    }
 }
 
 }  // namespace
@@ -1728,6 +1467,23 @@ static void launch_prefill(const ixg::PrefillParams& p, dim3 tgrid, dim3 cgrid, 
     }
 }
 
+// Whether the batch's sequences may run one workgroup per (sequence, up to two v heads of a q/k
+// head) (gdn_prefill_seq.hip): the pointers allow its vector accesses, the offsets its 32-bit
+// arithmetic, T' of one chunk's space its list of sequences, and there are enough workgroups
+// that batches of even lengths gain: at 12 and 16 sequences of U[1, 2048] tokens 16 q/k and 32 v heads
+// took 579 and 511 us against 662 and 768 us in windows, at 8 605 against 623, at 4 571 against 301; 16
+// and 48 heads (two workgroups per q/k head) 339 against 438 at 6; 8 and 16 heads 574 against 786
+// at 24, 590 against 566 at 16. Which of the sequences then do is decided on the device, from
+// their lengths (plan_kernel).
+constexpr long long kSeqWorkgroups = 176;
+static bool by_sequence(const ixg::PrefillParams& p, const ixg::OutGate& g, bool gated) {
+    auto on = [](const void* q, uintptr_t a) { return (reinterpret_cast<uintptr_t>(q) & (a - 1)) == 0; };
+    if (p.single || p.L.C >= 1 << 22 || p.n_seq > ixg::kTriFragBytes / 4 * p.L.h_v) return false;
+    if (!on(p.o_win ? nullptr : p.o, 16) || !on(p.o_bf16, 8)) return false;
+    if (gated && !(on(g.z, 8) && on(g.nrm, 16) && on(g.y, 16) && on(g.y_bf16, 8) && on(g.y_q8_1, 4))) return false;
+    return p.n_seq * ixg::seq_workgroups(p.L) >= kSeqWorkgroups;
+}
+
 static hipError_t prefill_impl(const ix_gdn_cfg* cfg, int n_seq, int total_T, const int32_t* cu_seqlens,
                                const uint16_t* x, uint16_t* conv_state, const uint16_t* conv_w, const uint16_t* a,
                                const uint16_t* b, const float* A_log, const float* dt_bias, float* state, float* o,
@@ -1770,16 +1526,31 @@ static hipError_t prefill_impl(const ix_gdn_cfg* cfg, int n_seq, int total_T, co
     p.o_win = gwin;
     if (gwin) p.o = reinterpret_cast<float*>(static_cast<char*>(workspace) + need);   // the norm's input
 
-    // Chain workgroups: (v head, strip, group), G groups splitting each window's chunks at
-    // sequence starts; one group while the h_v * 8 (head, strip) runs fill every CU.
+    const OutGate og = make_out_gate(gate);
+    const bool silu = cfg->conv_act == IX_GDN_ACT_SILU;
+    p.by_seq = by_sequence(p, og, gate != nullptr);
+    if (p.by_seq) {
+        // Measured: a chunk of a workgroup's walk 18.3 us with two heads, 12.2 with one (19 and 13 with
+        // the GPU full); in windows 3.3 us per chunk at 32 v heads, more or less in proportion.
+        const float one = cfg->h_v > cfg->h_k ? 18.3f : 12.2f;
+        p.cost_seq = one;
+        p.cost_work = 1.05f * one * (float)seq_workgroups(p.L) / (float)device_cu_count(s);
+        p.cost_win = 3.3f * (float)cfg->h_v / 32.0f;
+    }
+    if (!p.single) hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, p);
+    if (p.by_seq) {
+        PrefillParams q = p;
+        if (gwin) q.o = nullptr;
+        launch_prefill_seq(q, gate ? &og : nullptr, silu, s);
+    }
+
+    // The rest, or everything: chunk kernel and chain per window. Chain workgroups: (v head, strip,
+    // group), G groups splitting each window's chunks at sequence starts; one group while the
+    // h_v * 8 (head, strip) runs fill every CU.
     p.G = 1;
     if (!p.single) p.G = std::max(1, std::min(n_seq, ixg::device_cu_count(s) / (cfg->h_v * kStrips)));
-
-    if (!p.single) hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, p);
     const long long groups = ((long long)p.G * cfg->h_v + 7) / 8;
     const dim3 cgrid((unsigned)(groups * 8 * kStrips)), cblock(kChainWaves * kWave);
-    const bool silu = cfg->conv_act == IX_GDN_ACT_SILU;
-    const OutGate og = make_out_gate(gate);
     // Windows run in stream order: each chain resumes from the state and conv history the
     // previous one left; a window past the last chunk finds nothing to do.
     for (size_t cb = 0; cb < NCmax; cb += W) {
@@ -1791,11 +1562,12 @@ static hipError_t prefill_impl(const ix_gdn_cfg* cfg, int n_seq, int total_T, co
             case 3: launch_prefill<3>(p, tgrid, cgrid, cblock, silu, s); break;
             default: launch_prefill<4>(p, tgrid, cgrid, cblock, silu, s); break;
         }
-        if (gwin)
-            hipLaunchKernelGGL(out_gate_window_kernel, dim3((unsigned)(((long long)p.W * kChunk * cfg->h_v + 3) / 4)),
+        if (gwin || (gate && p.by_seq))
+            hipLaunchKernelGGL(out_gate_window_kernel,
+                               dim3((unsigned)std::min<long long>(((long long)p.W * kChunk * cfg->h_v + 3) / 4, kGateBlocks)),
                                dim3(256), 0, s, p, og);
     }
-    if (gate && !gwin)
+    if (gate && !gwin && !p.by_seq)
         hipLaunchKernelGGL(out_gate_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, p.o, og, rows);
     return hipGetLastError();
 }

@@ -58,6 +58,18 @@ __device__ __forceinline__ float wave_sum(float v) {
     return pair_sum32(pair_sum16(row_sum16(v)));
 }
 
+// Inclusive sum over lanes 0 .. l: shifts by 1, 2, 4, 8 within each 16-lane row, then each odd row
+// adds lane 15 of the row before it and the upper half adds lane 31 (DPP throughout, no LDS).
+__device__ __forceinline__ float wave_scan(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xF, 0xF, true));   // row_shr:1
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x112, 0xF, 0xF, true));   // row_shr:2
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xF, 0xF, true));   // row_shr:4
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xF, 0xF, true));   // row_shr:8
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));  // row_bcast:15
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));  // row_bcast:31
+    return v;
+}
+
 // Sixteen 64-lane sums at once, as a reduce-scatter: at lane distance 32, 16, 8 and 4 each
 // step exchanges half of the remaining partial sums with the partner lane (which keeps the
 // other half), so no partial sum is formed twice; the last two steps add within each quad.
@@ -128,5 +140,11 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 // Scalar math with the reference's definitions (src/ix_gdn.cu:22-23).
 __device__ __forceinline__ float softplus_f(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// sigmoid and SiLU on the hardware exp and reciprocal (1 ulp each; relative error below 1e-6 for
+// |x| < 10, and the limits 0 and 1 beyond fp32's exp range), for kernels that evaluate one per
+// output: 4 instructions against about 25.
+__device__ __forceinline__ float sigmoid_fast(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
+__device__ __forceinline__ float silu_f(float x) { return x * sigmoid_fast(x); }
 
 }  // namespace ixg

@@ -1,0 +1,81 @@
+"""Prefill batches with many sequences (gdn_prefill_seq.hip): one workgroup per sequence and one or
+two v heads, against the oracle, with lengths around the chunk's and its tiles' edges.
+
+Tolerances as in test_prefill_gpu.py (outputs 1e-3 absolute, state max|d|/max|ref| 1e-4, conv state
+and bf16 rounding exact); y against the norm of the double outputs 1e-4 (test_gated_gpu.py's
+end-to-end bound); q8_1 bytes equal the separate quantiser's.
+"""
+import numpy as np
+import pytest
+
+import baloon_amd as bx
+import oracle
+from oracle import bf16, inputs
+from tests.common import NT, TOL_O_ABS, TOL_STATE_REL, dev, host, state_from_dev, state_to_dev
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [0, 1, 2, 3, 4, 15, 16, 17, 31, 33, 48, 63, 64, 65, 66, 67, 80, 127, 128, 129, 130]
+
+
+def run(cfg, cu, tok, p, st, gate=None, window=None):
+    import torch
+    n, T = len(cu) - 1, tok["x"].shape[0]
+    size = bx.ix_gdn_prefill_workspace_size if gate is None else bx.ix_gdn_prefill_gated_workspace_size
+    need = size(cfg, n, T) if window is None else bx.ix_gdn_prefill_window_workspace_size(cfg, n, T, window,
+                                                                                          gate is not None)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    d_cs, d_st = dev(st["conv_state"]), state_to_dev(st["state"])
+    o = torch.full((T, cfg.h_v, cfg.d_v), float("nan"), device="cuda")
+    ob = torch.zeros(T, cfg.h_v, cfg.d_v, dtype=torch.bfloat16, device="cuda")
+    args = (cfg, n, T, dev(np.asarray(cu, np.int32)), dev(tok["x"]), d_cs, dev(p["w"]), dev(tok["a"]), dev(tok["b"]),
+            dev(p["A_log"]), dev(p["dt_bias"]), d_st)
+    if gate is None:
+        assert bx.ix_gdn_prefill(*args, o=o, o_bf16=ob, workspace=ws, workspace_bytes=need) == 0
+        torch.cuda.synchronize()
+        return host(d_cs), state_from_dev(d_st), host(o), host(ob)
+    y = torch.full((T, cfg.h_v, cfg.d_v), float("nan"), device="cuda")
+    yb = torch.zeros(T, cfg.h_v, cfg.d_v, dtype=torch.bfloat16, device="cuda")
+    yq = torch.zeros(T * cfg.h_v * cfg.d_v // 32 * 36, dtype=torch.uint8, device="cuda")
+    og = bx.out_gate(dev(gate["z"]), dev(gate["nrm"]), 1e-6, y, yb, yq)
+    assert bx.ix_gdn_prefill_gated(*args, gate=og, workspace=ws, workspace_bytes=need) == 0
+    torch.cuda.synchronize()
+    q = torch.zeros_like(yq)
+    assert bx.ix_q8_1_quantize(y, q, y.numel()) == 0
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(host(yq), host(q))
+    return host(d_cs), state_from_dev(d_st), host(y), host(yb)
+
+
+@pytest.mark.parametrize("kw,n", [
+    (dict(h_k=4, h_v=8), 45),                                  # two heads a workgroup
+    (dict(h_k=2, h_v=6, head_map=1, conv_act=1), 45),          # an odd count: the last half repeats a head
+    (dict(h_k=3, h_v=3, conv_act=1), 60),                      # one head a workgroup
+    (dict(h_k=2, h_v=5, d_conv=3), 60),                        # modulo pairing, uneven: 3 and 2 heads
+    (dict(h_k=4, h_v=2, d_conv=2), 45),                        # q/k heads without v heads
+    (dict(h_k=4, h_v=8, head_map=1, conv_act=1, q_scale=128 ** -0.5), 45),
+])
+@pytest.mark.parametrize("longest", [130, 1500])
+def test_many_sequences(kw, n, longest):
+    # longest = 1500: one sequence that the plan leaves to the windows among short ones.
+    cfg = bx.make_cfg(**kw)
+    lens = (EDGES * 3)[:n]
+    lens[7] = longest
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, seed = int(cu[-1]), inputs.seed_for(4) + 301 + n + longest
+    p, tok = inputs.layer_params(cfg, seed), inputs.token_inputs(cfg, seed, T)
+    st, g = inputs.initial_states(cfg, seed, n), inputs.out_gate_inputs(cfg, seed, T)
+    rcs, rs, ro = oracle.prefill(cfg, cu, tok["x"], st["conv_state"], p["w"], tok["a"], tok["b"], p["A_log"],
+                                 p["dt_bias"], st["state"], nthreads=NT)
+    cs, s, o, ob = run(cfg, cu, tok, p, st)
+    np.testing.assert_array_equal(cs, rcs)
+    assert oracle.rel_err(s, rs) <= TOL_STATE_REL
+    assert float(np.max(np.abs(o - ro))) <= TOL_O_ABS
+    np.testing.assert_array_equal(ob, bf16.from_f32(o))
+    gcs, gs, y, yb = run(cfg, cu, tok, p, st, g)
+    np.testing.assert_array_equal(gcs, cs)
+    np.testing.assert_array_equal(gs, s)                       # the norm changes no state
+    assert oracle.rel_err(y, oracle.gated_out(ro, g["z"], g["nrm"], 1e-6)) <= 1e-4
+    np.testing.assert_array_equal(yb, bf16.from_f32(y))
+    for a, b in zip((gcs, gs, y, yb), run(cfg, cu, tok, p, st, g, window=2)):
+        np.testing.assert_array_equal(a, b)                    # whatever the workspace
