@@ -8,7 +8,8 @@
 // z [B][h_v][d_v], and the gate and beta logits a, b [B][h_v]. This is the step to the left
 // of the recurrence that the reference runs as per-token bf16 GEMVs.
 //
-// At decode batch sizes the product is a skinny GEMM that streams W once from HBM (about 2
+// Prompts (many rows) run on larger tiles, in_proj_tile_kernel below; this is the decode batches'
+// kernel. At decode batch sizes the product is a skinny GEMM that streams W once from HBM (about 2
 // FLOP per weight byte at B = 64), so the work is moving bytes, not MFMA throughput. One
 // workgroup owns a 64 x 64 output tile over the whole of K. Two producer waves copy 64-k
 // stages of the tile's 64 activation rows (one wave) and 64 weight rows (the other) into a
@@ -23,6 +24,8 @@
 // each lane fetches. The summation order over K is fixed, so results do not depend on
 // timing.
 #include "gdn_common.h"
+
+#include <algorithm>
 
 namespace ixg {
 namespace {
@@ -53,6 +56,7 @@ struct InProj {
     uint16_t* b;                // [B][h_v]
     float* y;                   // [B][N] fp32, or null
     int B, K, N, C, Z, hv;
+    int n0;                     // first column of this launch
 };
 
 __device__ __forceinline__ void store_out(const InProj& p, int row, int col, float v) {
@@ -84,7 +88,7 @@ __global__ void __launch_bounds__((kCons + kProd) * kWave) in_proj_kernel(const 
 
     const int lane = threadIdx.x & (kWave - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int n0 = blockIdx.x * kNt, m0 = blockIdx.y * kMt;
+    const int n0 = p.n0 + blockIdx.x * kNt, m0 = blockIdx.y * kMt;
     const int nst = p.K / kKd;
 
     if (w >= kCons) {
@@ -180,6 +184,164 @@ __global__ void __launch_bounds__((kCons + kProd) * kWave) in_proj_kernel(const 
             }
 }
 
+// ---------------------------------------------------------------------------------------
+// Many rows (prompts): the product is bound by the matrix cores, and 64 x 64 tiles re-read each
+// operand so often that they ran at 402 TFLOP/s (4096 rows, hidden 2048, N = 12,352: 516 us). Here a
+// workgroup owns a BM x BN tile, its waves 2 x BN / 64 of them in accumulators (256 x 256 on 8 waves
+// of 128 x 64, or 128 x 128 on 4 of 64 x 64, two workgroups per CU), so that an operand row read from
+// LDS serves 64 or 128 columns. Stages of 64 k go through registers into one of two LDS buffers:
+// the loads of stage s + 2 and the LDS writes of stage s + 1 are issued ahead of stage s's products.
+// The tile columns are whole tiles of x and z (their width is a multiple of 128); in_proj_kernel
+// takes the rest. Outputs leave through LDS as whole row segments, 16 bytes a lane. Tiles are
+// numbered so that an XCD (workgroup index mod 8) works on a compact block: 8 row tiles, column by
+// column.
+// ---------------------------------------------------------------------------------------
+template <int BM, int BN>
+struct Tile {
+    static constexpr int kWavesM = 2, kWavesN = BN / 64, kWaves = kWavesM * kWavesN;
+    static constexpr int kThreads = kWaves * kWave;
+    static constexpr int kMT = BM / kWavesM / 16, kNT = 4;             // 16 x 16 tiles per wave
+    static constexpr int kBuf = (BM + BN) * kRowB;                     // one stage
+    static constexpr int kChunks = (BM + BN) * 8 / kThreads;           // 16-byte chunks per thread and stage
+    static constexpr int kOutRow = BN * 2 + 16;                        // bytes of an output row in LDS
+    static constexpr int kLds = 2 * kBuf > BM / 2 * kOutRow ? 2 * kBuf : BM / 2 * kOutRow;
+};
+
+template <int BM, int BN>
+__global__ void __launch_bounds__((Tile<BM, BN>::kThreads)) __attribute__((amdgpu_waves_per_eu(2)))
+in_proj_tile_kernel(const InProj p, int mt, int nt) {
+    using T = Tile<BM, BN>;
+    __shared__ __align__(16) uint8_t lds[T::kLds];
+    const int total = mt * nt, share = (total + 7) / 8;
+    const int id = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= share || id >= total) return;
+    const int grp = id / (8 * nt), gm = min(8, mt - 8 * grp), in = id - grp * 8 * nt;
+    const int m0 = (8 * grp + in % gm) * BM, n0 = in / gm * BN;
+
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), li = lane & 15, lg = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int wm = (w & 1) * (BM / 2), wn = (w >> 1) * 64;
+    const int nst = p.K / kKd;
+
+    // Chunk c of rows r0, r0 + T / 8, ...: activation rows, then weight rows (rows past the batch
+    // repeat its last one; their results are never stored).
+    const int c = tid & 7, r0 = tid >> 3;
+    const uint8_t* src[T::kChunks];
+#pragma unroll
+    for (int i = 0; i < T::kChunks; ++i) {
+        const int r = r0 + i * (T::kThreads / 8);
+        const bool act = i * (T::kThreads / 8) < BM;
+        const int row = act ? min(m0 + r, p.B - 1) : n0 + r - BM;
+        src[i] = reinterpret_cast<const uint8_t*>(act ? p.h : p.w) + (size_t)row * p.K * 2 + c * 16;
+    }
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 st[T::kChunks];
+    auto load = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < T::kChunks; ++i) st[i] = *reinterpret_cast<const u32x4*>(src[i] + (size_t)s * kRowB);
+    };
+    const int wo = ring_off(r0, c);                              // r0 + multiples of 8: the same swizzle
+    auto put = [&](int s) {
+        uint8_t* b = lds + (s & 1) * T::kBuf + wo;
+#pragma unroll
+        for (int i = 0; i < T::kChunks; ++i) *reinterpret_cast<u32x4*>(b + i * (T::kThreads / 8) * kRowB) = st[i];
+    };
+
+    f32x4 acc[T::kMT][T::kNT];
+#pragma unroll
+    for (int i = 0; i < T::kMT; ++i)
+#pragma unroll
+        for (int j = 0; j < T::kNT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int ao[2], bo[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        ao[ks] = ring_off(wm + li, 4 * ks + lg);
+        bo[ks] = BM * kRowB + ring_off(wn + li, 4 * ks + lg);
+    }
+
+    load(0);
+    put(0);
+    if (nst > 1) load(1);
+    for (int s = 0; s < nst; ++s) {
+        lds_barrier();                                           // stage s written; stage s - 1 read
+        if (s + 1 < nst) put(s + 1);
+        if (s + 2 < nst) load(s + 2);
+        const uint8_t* b = lds + (s & 1) * T::kBuf;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            bf16x8 av[T::kMT], bv[T::kNT];
+#pragma unroll
+            for (int j = 0; j < T::kNT; ++j) bv[j] = *reinterpret_cast<const bf16x8*>(b + bo[ks] + j * 16 * kRowB);
+#pragma unroll
+            for (int i = 0; i < T::kMT; ++i) av[i] = *reinterpret_cast<const bf16x8*>(b + ao[ks] + i * 16 * kRowB);
+#pragma unroll
+            for (int i = 0; i < T::kMT; ++i)
+#pragma unroll
+                for (int j = 0; j < T::kNT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // Outputs, half of the tile's rows at a time (the waves of one wm).
+    const bool isz = n0 >= p.C;
+    const int width = isz ? p.Z : p.C, col0 = isz ? n0 - p.C : n0;
+    uint16_t* out = isz ? p.z : p.x;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        lds_barrier();
+        if ((w & 1) == half) {
+#pragma unroll
+            for (int i = 0; i < T::kMT; ++i)
+#pragma unroll
+                for (int j = 0; j < T::kNT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        *reinterpret_cast<uint16_t*>(lds + (16 * i + 4 * lg + r) * T::kOutRow + 2 * (wn + 16 * j + li)) =
+                            f32_to_bf16(acc[i][j][r]);
+        }
+        lds_barrier();
+        constexpr int kPerRow = BN / 8, kRows = T::kThreads / kPerRow;
+#pragma unroll
+        for (int i = 0; i < BM / 2 / kRows; ++i) {
+            const int r = i * kRows + tid / kPerRow, cc = tid % kPerRow, row = m0 + half * (BM / 2) + r;
+            const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * T::kOutRow + 16 * cc);
+            if (row < p.B) *reinterpret_cast<u32x4*>(out + (size_t)row * width + col0 + 8 * cc) = v;
+        }
+    }
+}
+
+template <int BM, int BN>
+void launch_tiles(const InProj& p, int cols, hipStream_t s) {
+    const int mt = (p.B + BM - 1) / BM, nt = cols / BN;
+    const dim3 grid(8u * (unsigned)((mt * nt + 7) / 8)), block(Tile<BM, BN>::kThreads);
+    hipLaunchKernelGGL((in_proj_tile_kernel<BM, BN>), grid, block, 0, s, p, mt, nt);
+}
+
+// Columns that a tile kernel has been launched for (0: none). The bf16 pieces only, 16-byte row
+// segments, tiles not across the x | z boundary; and where the tiles cost less than 64 x 64 ones for the
+// whole product. Prices in us at K = 2048 on 256 CUs (they scale with K; 8 us of the tiles' stay
+// the same: the launch for the remaining columns), as measured for 100 to 4096 rows, N = 3,088 to
+// 12,352 and K = 1024 to 2048: 0.048 per 64 x 64 tile (4096 rows, N = 12,352: 513 us); two 128 x 128 tiles per CU in
+// 39, one in 26 (512 rows: 50 us against 70; 2048 rows: 128); a 256 x 256 tile per CU in 58 (4096 rows:
+// 196 us, 1,055 TFLOP/s, against 242 with 128 x 128).
+int tile_columns(const InProj& p, hipStream_t s) {
+    auto on16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    if (p.y || !on16(p.x) || !on16(p.z)) return 0;
+    const long long cu = device_cu_count(s), all = p.C + p.Z;
+    auto tiles = [&](long long cols, int t) { return ((p.B + t - 1) / t) * (cols / t); };
+    const double k = p.K / 2048.0;
+    const long long w128 = tiles(all, 128), half = (w128 + cu - 1) / cu;       // rounds of one tile per CU
+    const double c64 = 0.048 * 256 / cu * ((p.B + 63) / 64) * ((p.N + 63) / 64);
+    const double c128 = 39.0 * (half / 2) + 26.0 * (half & 1);
+    const double c256 = p.C % 256 ? 1e30 : 58.0 * ((tiles(all, 256) + cu - 1) / cu);
+    if (k * c64 <= 8.0 + k * std::min(c128, c256)) return 0;
+    if (c256 < c128) {
+        launch_tiles<256, 256>(p, (int)(all / 256 * 256), s);
+        return (int)(all / 256 * 256);
+    }
+    launch_tiles<128, 128>(p, (int)all, s);
+    return (int)all;
+}
+
 }  // namespace
 }  // namespace ixg
 
@@ -208,7 +370,8 @@ extern "C" hipError_t ix_gdn_in_proj(const ix_gdn_cfg* cfg, int B, int hidden, c
     p.Z = cfg->h_v * cfg->d_v;
     p.hv = cfg->h_v;
     p.N = p.C + p.Z + 2 * p.hv;
-    const dim3 grid((unsigned)((p.N + kNt - 1) / kNt), (unsigned)((B + kMt - 1) / kMt));
+    p.n0 = tile_columns(p, s);
+    const dim3 grid((unsigned)((p.N - p.n0 + kNt - 1) / kNt), (unsigned)((B + kMt - 1) / kMt));
     hipLaunchKernelGGL(in_proj_kernel, grid, dim3((kCons + kProd) * kWave), 0, s, p);
     return hipGetLastError();
 }
