@@ -112,7 +112,7 @@ gemv_block_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w
 //   Q8_0 block: fp16 scale d, 32 int8 (34 bytes, 2-byte aligned); w [n_out][n_in/32]
 //   q8_1 block: fp16 d, fp16 s (sum, unused by Q8_0), 32 int8 (36 bytes); x [ncols][n_in/32]
 // y[c][r] = sum over blocks of d_w * d_x * (integer dot of the 32 pairs).
-// One wave per row; each block is split over two lanes (16 values each: four v_dot4_i32_i8),
+// Few rows, or long ones: one wave per row; each block is split over two lanes (16 values each: four v_dot4_i32_i8),
 // the two integer halves are added exactly, then scaled once per block. Each column's sum is
 // computed by the same code whatever the number of columns launched.
 // ---------------------------------------------------------------------------------------
@@ -158,11 +158,80 @@ mmvq_q8_0_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ x, f
     }
 }
 
+// Many rows: with the activations read from memory for every row, their loads (36-byte stride, 16 bytes a
+// lane: some 36 cycles of the vector cache each) bound the product, 2.5 us per column of 4096 x
+// 6144. Here a workgroup keeps the blocks of all its columns in LDS (codes as two planes of 16 bytes
+// per block, scales as floats; one or two cycles per 128 bytes) and its 8 waves walk rows, a lane
+// one whole block per step. 4096 -> 6144 with 1, 2, 4, 8 columns: 7.1, 9.6, 12.9, 19.3 us -> 6.0, 6.2, 6.7,
+// 8.1 (26.7 MB of weights: 4.5 to 3.3 TB/s).
+constexpr int kQLdsThreads = 512, kQLdsWaves = kQLdsThreads / kWave;
+template <int NC>
+__global__ void __launch_bounds__(kQLdsThreads)
+mmvq_q8_0_lds_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ x, float* __restrict__ y, int n_in,
+                     int n_out) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));   // Q8_0 codes: 2-byte aligned
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), nb = n_in / 32;
+    u32x4* xq = reinterpret_cast<u32x4*>(lds);                                   // [NC][2][nb]
+    float* xd = reinterpret_cast<float*>(lds + (size_t)NC * 32 * nb);            // [NC][nb]
+    for (int i = tid; i < NC * nb; i += kQLdsThreads) {
+        const uint32_t* b = reinterpret_cast<const uint32_t*>(x + (size_t)i * kQ81Bytes);
+        const int c = i / nb, kb = i - c * nb;
+        xd[i] = half_to_f32((uint16_t)b[0]);
+        xq[(2 * c) * nb + kb] = u32x4{b[1], b[2], b[3], b[4]};
+        xq[(2 * c + 1) * nb + kb] = u32x4{b[5], b[6], b[7], b[8]};
+    }
+    __syncthreads();
+    for (int row = (int)blockIdx.x * kQLdsWaves + tid / kWave; row < n_out; row += (int)gridDim.x * kQLdsWaves) {
+        const uint8_t* wr = w + (size_t)row * nb * kQ80Bytes;
+        float acc[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c] = 0.0f;
+#pragma unroll 2
+        for (int kb = lane; kb < nb; kb += kWave) {
+            const uint8_t* wb = wr + (size_t)kb * kQ80Bytes;
+            const u32x4_a2 w0 = *reinterpret_cast<const u32x4_a2*>(wb + 2), w1 = *reinterpret_cast<const u32x4_a2*>(wb + 18);
+            const float dw = half_to_f32(*reinterpret_cast<const uint16_t*>(wb));
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const u32x4 x0 = xq[(2 * c) * nb + kb], x1 = xq[(2 * c + 1) * nb + kb];
+                int s = 0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s = __builtin_amdgcn_sdot4((int)w0[i], (int)x0[i], s, false);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s = __builtin_amdgcn_sdot4((int)w1[i], (int)x1[i], s, false);
+                acc[c] = fmaf(dw * xd[c * nb + kb], (float)s, acc[c]);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const float v = wave_sum(acc[c]);
+            if (lane == 0) y[(size_t)c * n_out + row] = v;
+        }
+    }
+}
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 inline bool vec_rows(const uint16_t* x, const uint16_t* w, long long n_in) {
     return n_in % 8 == 0 && aligned16(x) && aligned16(w);
 }
 inline unsigned row_blocks(long long n_out) { return (unsigned)((n_out + kRowsPerBlock - 1) / kRowsPerBlock); }
+
+// The LDS kernel from 1024 rows (512 rows: 2.1 against 2.0 us with one column) while 8 columns'
+// blocks fit 64 KiB (n_in <= 7264), two workgroups per CU (one: 9.6 against 8.1 us with 8 columns of 4096 ->
+// 6144, four: 9.3). The choice depends on the matrix alone, so that a column's result does not
+// depend on the number of columns.
+template <int NC>
+void launch_q8_0(const uint8_t* w, const uint8_t* x, float* y, int n_in, int n_out, hipStream_t s) {
+    const int nb = n_in / 32;
+    if (n_out < 1024 || 8LL * kQ81Bytes * nb > 65536) {
+        hipLaunchKernelGGL(mmvq_q8_0_kernel<NC>, dim3(row_blocks(n_out)), dim3(kGemvThreads), 0, s, w, x, y, n_in, n_out);
+        return;
+    }
+    const int grid = std::min((n_out + kQLdsWaves - 1) / kQLdsWaves, 2 * device_cu_count(s));
+    hipLaunchKernelGGL(mmvq_q8_0_lds_kernel<NC>, dim3((unsigned)grid), dim3(kQLdsThreads), (unsigned)(NC * kQ81Bytes * nb), s,
+                       w, x, y, n_in, n_out);
+}
 
 // q8_1 quantiser: x [n] fp32 -> [n/32] q8_1 blocks; each wave takes 64 consecutive values
 // (two blocks, one per half wave) per step, through the same q81_store as the gated epilogues.
@@ -241,16 +310,15 @@ extern "C" hipError_t ix_mmvq_q8_0(const void* weights, const void* x_q8_1, floa
         return hipErrorInvalidValue;                         // block alignment of the formats
     const auto* w = static_cast<const uint8_t*>(weights);
     const auto* x = static_cast<const uint8_t*>(x_q8_1);
-    const dim3 grid(row_blocks(n_out)), block(kGemvThreads);
     switch (ncols) {
-        case 1: hipLaunchKernelGGL(mmvq_q8_0_kernel<1>, grid, block, 0, s, w, x, y, n_in, n_out); break;
-        case 2: hipLaunchKernelGGL(mmvq_q8_0_kernel<2>, grid, block, 0, s, w, x, y, n_in, n_out); break;
-        case 3: hipLaunchKernelGGL(mmvq_q8_0_kernel<3>, grid, block, 0, s, w, x, y, n_in, n_out); break;
-        case 4: hipLaunchKernelGGL(mmvq_q8_0_kernel<4>, grid, block, 0, s, w, x, y, n_in, n_out); break;
-        case 5: hipLaunchKernelGGL(mmvq_q8_0_kernel<5>, grid, block, 0, s, w, x, y, n_in, n_out); break;
-        case 6: hipLaunchKernelGGL(mmvq_q8_0_kernel<6>, grid, block, 0, s, w, x, y, n_in, n_out); break;
-        case 7: hipLaunchKernelGGL(mmvq_q8_0_kernel<7>, grid, block, 0, s, w, x, y, n_in, n_out); break;
-        default: hipLaunchKernelGGL(mmvq_q8_0_kernel<8>, grid, block, 0, s, w, x, y, n_in, n_out); break;
+        case 1: launch_q8_0<1>(w, x, y, n_in, n_out, s); break;
+        case 2: launch_q8_0<2>(w, x, y, n_in, n_out, s); break;
+        case 3: launch_q8_0<3>(w, x, y, n_in, n_out, s); break;
+        case 4: launch_q8_0<4>(w, x, y, n_in, n_out, s); break;
+        case 5: launch_q8_0<5>(w, x, y, n_in, n_out, s); break;
+        case 6: launch_q8_0<6>(w, x, y, n_in, n_out, s); break;
+        case 7: launch_q8_0<7>(w, x, y, n_in, n_out, s); break;
+        default: launch_q8_0<8>(w, x, y, n_in, n_out, s); break;
     }
     return hipGetLastError();
 }
