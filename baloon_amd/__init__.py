@@ -8,7 +8,8 @@ error behaviour -- every call returns a ``hipError_t`` code (0 = success), with
 
 PyTorch is only plumbing here: tensors supply device memory and the current stream. Every
 tensor argument must live on the GPU; the functions pass raw device pointers to the C ABI.
-There is no CPU fallback: if the library is missing, :func:`lib` raises.
+There is no CPU fallback: if the library is missing, :func:`lib` raises. The launchers' arguments
+are converted by the extension ``_bind`` (csrc/bind.cpp); the other symbols are bound with ctypes.
 """
 from __future__ import annotations
 
@@ -121,6 +122,7 @@ def lib() -> ctypes.CDLL:
         fn = getattr(L, name)
         fn.argtypes = args
         fn.restype = res
+        _bind.bind(name, ctypes.cast(fn, P).value)
     _lib = L
     return L
 
@@ -143,6 +145,34 @@ def _stream(s) -> int | None:
     return getattr(s, "cuda_stream", s)
 
 
+class _Unbuilt:
+    """Stands for the extension until it has been built."""
+
+    def __getattr__(self, name):
+        return getattr(_import_bind(), name)
+
+
+def _import_bind():
+    global _bind
+    import importlib
+
+    import torch  # noqa: F401  (before _bind, which uses its libraries)
+    try:
+        m = importlib.import_module("._bind", __name__)
+    except ImportError as e:
+        raise RuntimeError(f"{PKG}/_bind.so is missing or does not load: build it with "
+                           "`python -m baloon_amd.build`") from e
+    m.setup(lib, _ptr, Cfg, OutGate)
+    _bind = m
+    return m
+
+
+try:
+    _import_bind()
+except RuntimeError:
+    _bind = _Unbuilt()
+
+
 def check(name: str, code: int) -> None:
     if code != HIP_SUCCESS:
         raise IxGdnError(name, code)
@@ -151,24 +181,23 @@ def check(name: str, code: int) -> None:
 # ---- legacy entry points (src/ix_gdn.cu:108-136), return hipError_t --------------------------
 
 def ix_gdn_step(state, q, k, v, gate, beta, o, S, h_k, h_v, s=None) -> int:
-    return lib().ix_gdn_step(_ptr(state), _ptr(q), _ptr(k), _ptr(v), _ptr(gate), _ptr(beta), _ptr(o),
-                             S, h_k, h_v, _stream(s))
+    return _bind.ix_gdn_step(state, q, k, v, gate, beta, o, S, h_k, h_v, s)
 
 
 def ix_gdn_conv_step(conv_state, x, kW, out, channels, d_conv, s=None) -> int:
-    return lib().ix_gdn_conv_step(_ptr(conv_state), _ptr(x), _ptr(kW), _ptr(out), channels, d_conv, _stream(s))
+    return _bind.ix_gdn_conv_step(conv_state, x, kW, out, channels, d_conv, s)
 
 
 def ix_gdn_l2_norm(x, rows, cols, eps, s=None) -> int:
-    return lib().ix_gdn_l2_norm(_ptr(x), rows, cols, eps, _stream(s))
+    return _bind.ix_gdn_l2_norm(x, rows, cols, eps, s)
 
 
 def ix_gdn_beta_gate(beta, h_v, s=None) -> int:
-    return lib().ix_gdn_beta_gate(_ptr(beta), h_v, _stream(s))
+    return _bind.ix_gdn_beta_gate(beta, h_v, s)
 
 
 def ix_gdn_out_norm(o, z, ssm_norm, y, h_v, S, eps, s=None) -> int:
-    return lib().ix_gdn_out_norm(_ptr(o), _ptr(z), _ptr(ssm_norm), _ptr(y), h_v, S, eps, _stream(s))
+    return _bind.ix_gdn_out_norm(o, z, ssm_norm, y, h_v, S, eps, s)
 
 
 # ---- fused layer entry points ------------------------------------------------------------------
@@ -184,9 +213,7 @@ def ix_gdn_decode(cfg: Cfg, B, x, conv_state, conv_w, a, b, A_log, dt_bias, stat
     state is [B][h_v][d_v][d_k] fp32 (each head's state stored column by column). workspace,
     if given, is a device buffer of ix_gdn_decode_workspace_size(cfg, B) bytes, zero-filled
     once (the calls keep its counters at zero); it selects the faster many-workgroup kernel."""
-    return lib().ix_gdn_decode(ctypes.byref(cfg), B, _ptr(x), _ptr(conv_state), _ptr(conv_w), _ptr(a), _ptr(b),
-                               _ptr(A_log), _ptr(dt_bias), _ptr(state), _ptr(o), _ptr(o_bf16), _ptr(workspace),
-                               _stream(s))
+    return _bind.ix_gdn_decode(cfg, B, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o, o_bf16, workspace, s)
 
 
 def ix_gdn_decode_noalloc(cfg: Cfg, B, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o=None, o_bf16=None,
@@ -194,9 +221,7 @@ def ix_gdn_decode_noalloc(cfg: Cfg, B, x, conv_state, conv_w, a, b, A_log, dt_bi
     """ix_gdn_decode without a workspace and without any allocation: the group counters live
     in a library-owned static device array (B * h_k <= 65536). Calls on one GPU must be
     ordered (they share the array)."""
-    return lib().ix_gdn_decode_noalloc(ctypes.byref(cfg), B, _ptr(x), _ptr(conv_state), _ptr(conv_w), _ptr(a),
-                                       _ptr(b), _ptr(A_log), _ptr(dt_bias), _ptr(state), _ptr(o), _ptr(o_bf16),
-                                       _stream(s))
+    return _bind.ix_gdn_decode_noalloc(cfg, B, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o, o_bf16, s)
 
 
 def ix_gdn_prefill_workspace_size(cfg: Cfg, n_seq: int, total_T: int) -> int:
@@ -205,9 +230,8 @@ def ix_gdn_prefill_workspace_size(cfg: Cfg, n_seq: int, total_T: int) -> int:
 
 def ix_gdn_prefill(cfg: Cfg, n_seq, total_T, cu_seqlens, x, conv_state, conv_w, a, b, A_log, dt_bias, state,
                    o=None, o_bf16=None, workspace=None, workspace_bytes=0, s=None) -> int:
-    return lib().ix_gdn_prefill(ctypes.byref(cfg), n_seq, total_T, _ptr(cu_seqlens), _ptr(x), _ptr(conv_state),
-                                _ptr(conv_w), _ptr(a), _ptr(b), _ptr(A_log), _ptr(dt_bias), _ptr(state), _ptr(o),
-                                _ptr(o_bf16), _ptr(workspace), workspace_bytes, _stream(s))
+    return _bind.ix_gdn_prefill(cfg, n_seq, total_T, cu_seqlens, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o,
+                                o_bf16, workspace, workspace_bytes, s)
 
 
 def out_gate(z, ssm_norm, eps, y=None, y_bf16=None, y_q8_1=None) -> OutGate:
@@ -219,10 +243,8 @@ def out_gate(z, ssm_norm, eps, y=None, y_bf16=None, y_q8_1=None) -> OutGate:
 def ix_gdn_decode_gated(cfg: Cfg, B, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o=None, o_bf16=None,
                         gate: OutGate | None = None, workspace=None, s=None) -> int:
     """ix_gdn_decode plus the gated RMS output norm of each (sequence, v head) in the same launch."""
-    g = ctypes.byref(gate) if gate is not None else None
-    return lib().ix_gdn_decode_gated(ctypes.byref(cfg), B, _ptr(x), _ptr(conv_state), _ptr(conv_w), _ptr(a),
-                                     _ptr(b), _ptr(A_log), _ptr(dt_bias), _ptr(state), _ptr(o), _ptr(o_bf16), g,
-                                     _ptr(workspace), _stream(s))
+    return _bind.ix_gdn_decode_gated(cfg, B, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o, o_bf16, gate,
+                                     workspace, s)
 
 
 def ix_gdn_prefill_gated_workspace_size(cfg: Cfg, n_seq: int, total_T: int) -> int:
@@ -240,11 +262,8 @@ def ix_gdn_prefill_gated(cfg: Cfg, n_seq, total_T, cu_seqlens, x, conv_state, co
                          o=None, o_bf16=None, gate: OutGate | None = None, workspace=None, workspace_bytes=0,
                          s=None) -> int:
     """ix_gdn_prefill plus the gated RMS output norm of every (token, v head) row."""
-    g = ctypes.byref(gate) if gate is not None else None
-    return lib().ix_gdn_prefill_gated(ctypes.byref(cfg), n_seq, total_T, _ptr(cu_seqlens), _ptr(x),
-                                      _ptr(conv_state), _ptr(conv_w), _ptr(a), _ptr(b), _ptr(A_log), _ptr(dt_bias),
-                                      _ptr(state), _ptr(o), _ptr(o_bf16), g, _ptr(workspace), workspace_bytes,
-                                      _stream(s))
+    return _bind.ix_gdn_prefill_gated(cfg, n_seq, total_T, cu_seqlens, x, conv_state, conv_w, a, b, A_log, dt_bias,
+                                      state, o, o_bf16, gate, workspace, workspace_bytes, s)
 
 
 def ix_gdn_window_record_size(cfg: Cfg, B: int, K: int) -> int:
@@ -254,24 +273,21 @@ def ix_gdn_window_record_size(cfg: Cfg, B: int, K: int) -> int:
 def ix_gdn_decode_window(cfg: Cfg, B, K, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o=None, o_bf16=None,
                          record=None, s=None) -> int:
     """Verify K draft tokens per sequence (x [B][K][C]); the states are read, not written."""
-    return lib().ix_gdn_decode_window(ctypes.byref(cfg), B, K, _ptr(x), _ptr(conv_state), _ptr(conv_w), _ptr(a),
-                                      _ptr(b), _ptr(A_log), _ptr(dt_bias), _ptr(state), _ptr(o), _ptr(o_bf16),
-                                      _ptr(record), _stream(s))
+    return _bind.ix_gdn_decode_window(cfg, B, K, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o, o_bf16, record,
+                                      s)
 
 
 def ix_gdn_decode_window_mfma(cfg: Cfg, B, K, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o=None,
                               o_bf16=None, record=None, s=None) -> int:
     """ix_gdn_decode_window on the matrix cores: outputs to fp32 rounding of the exact verify,
     the same record."""
-    return lib().ix_gdn_decode_window_mfma(ctypes.byref(cfg), B, K, _ptr(x), _ptr(conv_state), _ptr(conv_w),
-                                           _ptr(a), _ptr(b), _ptr(A_log), _ptr(dt_bias), _ptr(state), _ptr(o),
-                                           _ptr(o_bf16), _ptr(record), _stream(s))
+    return _bind.ix_gdn_decode_window_mfma(cfg, B, K, x, conv_state, conv_w, a, b, A_log, dt_bias, state, o, o_bf16,
+                                           record, s)
 
 
 def ix_gdn_commit_window(cfg: Cfg, B, K, accepted, x, record, conv_state, state, s=None) -> int:
     """Advance each sequence's states by its accepted prefix of the verified window."""
-    return lib().ix_gdn_commit_window(ctypes.byref(cfg), B, K, _ptr(accepted), _ptr(x), _ptr(record),
-                                      _ptr(conv_state), _ptr(state), _stream(s))
+    return _bind.ix_gdn_commit_window(cfg, B, K, accepted, x, record, conv_state, state, s)
 
 
 def layer_pointer_table(tensors):
@@ -306,24 +322,24 @@ def ix_gdn_commit_window_layers(cfg: Cfg, B, K, accepted, xs, records, conv_stat
 # ---- projections ----------------------------------------------------------------------------
 
 def ix_bf16_gemv(x, w, y, n_in, n_out, s=None) -> int:
-    return lib().ix_bf16_gemv(_ptr(x), _ptr(w), _ptr(y), n_in, n_out, _stream(s))
+    return _bind.ix_bf16_gemv(x, w, y, n_in, n_out, s)
 
 
 def ix_bf16_gemv_pair(x, w1, y1, n_out1, w2, y2, n_out2, n_in, s=None) -> int:
-    return lib().ix_bf16_gemv_pair(_ptr(x), _ptr(w1), _ptr(y1), n_out1, _ptr(w2), _ptr(y2), n_out2, n_in, _stream(s))
+    return _bind.ix_bf16_gemv_pair(x, w1, y1, n_out1, w2, y2, n_out2, n_in, s)
 
 
 def ix_bf16_gemv_split(x, w, y, n_in, n_out, threads_per_row, s=None) -> int:
-    return lib().ix_bf16_gemv_split(_ptr(x), _ptr(w), _ptr(y), n_in, n_out, threads_per_row, _stream(s))
+    return _bind.ix_bf16_gemv_split(x, w, y, n_in, n_out, threads_per_row, s)
 
 
 def ix_mmvq_q8_0(weights, x_q8_1, y, n_in, n_out, ncols, s=None) -> int:
-    return lib().ix_mmvq_q8_0(_ptr(weights), _ptr(x_q8_1), _ptr(y), n_in, n_out, ncols, _stream(s))
+    return _bind.ix_mmvq_q8_0(weights, x_q8_1, y, n_in, n_out, ncols, s)
 
 
 def ix_q8_1_quantize(x, y_q8_1, n, s=None) -> int:
     """q8_1 blocks (36 bytes per 32 values) of n fp32 values: the activation format of ix_mmvq_q8_0."""
-    return lib().ix_q8_1_quantize(_ptr(x), _ptr(y_q8_1), n, _stream(s))
+    return _bind.ix_q8_1_quantize(x, y_q8_1, n, s)
 
 
 def ix_gdn_in_proj_width(cfg: Cfg) -> int:
@@ -332,8 +348,7 @@ def ix_gdn_in_proj_width(cfg: Cfg) -> int:
 
 def ix_gdn_in_proj(cfg: Cfg, B, hidden, h, w, x, z, a, b, y=None, s=None) -> int:
     """[x | z | a | b] = h W^T for B rows: h [B][hidden], W [N][hidden] bf16 -> bf16 pieces."""
-    return lib().ix_gdn_in_proj(ctypes.byref(cfg), B, hidden, _ptr(h), _ptr(w), _ptr(x), _ptr(z), _ptr(a), _ptr(b),
-                                _ptr(y), _stream(s))
+    return _bind.ix_gdn_in_proj(cfg, B, hidden, h, w, x, z, a, b, y, s)
 
 
 def version() -> str:

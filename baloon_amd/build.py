@@ -1,6 +1,6 @@
-"""Build libixgdn.so (HIP, gfx950) in-tree with hipcc.
+"""Build libixgdn.so (HIP, gfx950) in-tree with hipcc, and _bind.so, the Python mirror's call path.
 
-    python -m baloon_amd.build           # compile every csrc/*.hip and link the library
+    python -m baloon_amd.build           # compile every csrc/*.hip and link the library; csrc/bind.cpp
 
 Each translation unit is compiled for gfx950 only, with packed-FP32 instruction selection
 disabled (-packed-fp32-ops), and with kernel resource-usage remarks captured to
@@ -22,6 +22,7 @@ CSRC = os.path.join(PKG, "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libixgdn.so")
+BIND = os.path.join(PKG, "_bind.so")
 RESOURCE_REPORT = os.path.join(BUILD, "resource_usage.txt")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -76,11 +77,34 @@ def _resource_summary(remarks: str) -> str:
     return "\n".join(out) + "\n"
 
 
+def _build_bind() -> None:
+    """_bind.so: host C++ against the Python and torch headers (csrc/bind.cpp)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc = [INCLUDE, sysconfig.get_paths()["include"], *include_paths(), os.path.join(rocm, "include")]
+    tmp = BIND + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[a for p in inc for a in ("-isystem", p)], os.path.join(CSRC, "bind.cpp"), "-o", tmp,
+           "-L", libs, "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"the Python binding failed to build:\n{r.stderr}")
+    os.replace(tmp, BIND)
+
+
 def build(verbose: bool = False) -> str:
     os.makedirs(BUILD, exist_ok=True)
     srcs = sources()
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        bind = ex.submit(_build_bind)
         results = list(ex.map(_compile, srcs))
+        bind.result()
     objs = [o for o, _ in results]
     remarks = "".join(r for _, r in results)
     with open(RESOURCE_REPORT, "w") as f:
