@@ -159,10 +159,10 @@ def _import_bind():
     import torch  # noqa: F401  (before _bind, which uses its libraries)
     try:
         m = importlib.import_module("._bind", __name__)
-    except ImportError as e:
+        m.setup(lib, _ptr, ctypes.Structure.__mro__[-2])      # the base of every ctypes type
+    except (ImportError, TypeError) as e:                      # TypeError: built from older sources
         raise RuntimeError(f"{PKG}/_bind.so is missing or does not load: build it with "
                            "`python -m baloon_amd.build`") from e
-    m.setup(lib, _ptr, Cfg, OutGate)
     _bind = m
     return m
 

@@ -7,7 +7,7 @@
 // 38 us for 16 us of kernels. Here an argument is read from the tensor's C++ object.
 //
 // Arguments are converted by the C parameter's type: pointers from tensors (on the GPU, contiguous)
-// or None, descriptions from the ctypes structures, the stream from None (torch's current one), a
+// or None, descriptions from ctypes structures, the stream from None (torch's current one), a
 // torch stream or an address. Anything but a plain torch.Tensor or Parameter goes through the
 // mirror's own _ptr, which refuses or reads it as before. The library's functions are found by
 // the mirror (lib()), which hands their addresses over.
@@ -26,8 +26,7 @@ namespace {
 
 PyObject* g_load = nullptr;     // lib(): loads the library and binds the addresses below
 PyObject* g_ptr = nullptr;      // _ptr()
-PyObject* g_cfg = nullptr;      // Cfg
-PyObject* g_gate = nullptr;     // OutGate
+PyObject* g_cdata = nullptr;    // the base of every ctypes type
 
 // Every converter returns with a Python error set if the argument does not fit.
 void* tensor_ptr(PyObject* o) {
@@ -51,13 +50,14 @@ long long integer(PyObject* o) {
     return (long long)v;
 }
 
+// Any ctypes instance of the C structure's size or more (a program may declare its own mirror of it).
 template <class T>
-const T* structure(PyObject* o, PyObject* type) {
-    const int is = PyObject_IsInstance(o, type);
+const T* structure(PyObject* o) {
+    const int is = PyObject_IsInstance(o, g_cdata);
     if (is < 0) return nullptr;
     Py_buffer b;
     if (!is) {
-        PyErr_Format(PyExc_TypeError, "expected %R, got %R", type, (PyObject*)Py_TYPE(o));
+        PyErr_Format(PyExc_TypeError, "expected a ctypes instance, got %R", (PyObject*)Py_TYPE(o));
         return nullptr;
     }
     if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) return nullptr;
@@ -91,12 +91,12 @@ struct Arg {                                                 // pointers to devi
 };
 template <>
 struct Arg<const ix_gdn_cfg*> {
-    static const ix_gdn_cfg* of(PyObject* o) { return structure<ix_gdn_cfg>(o, g_cfg); }
+    static const ix_gdn_cfg* of(PyObject* o) { return structure<ix_gdn_cfg>(o); }
 };
 template <>
 struct Arg<const ix_gdn_out_gate*> {
     static const ix_gdn_out_gate* of(PyObject* o) {
-        return o == Py_None ? nullptr : structure<ix_gdn_out_gate>(o, g_gate);
+        return o == Py_None ? nullptr : structure<ix_gdn_out_gate>(o);
     }
 };
 template <>
@@ -181,12 +181,12 @@ PyObject* bind(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
-// setup(lib, _ptr, Cfg, OutGate)
+// setup(lib, _ptr, ctypes' base type)
 PyObject* setup(PyObject*, PyObject* args) {
-    PyObject *l, *p, *c, *g;
-    if (!PyArg_ParseTuple(args, "OOOO", &l, &p, &c, &g)) return nullptr;
-    Py_INCREF(l); Py_INCREF(p); Py_INCREF(c); Py_INCREF(g);
-    g_load = l; g_ptr = p; g_cfg = c; g_gate = g;
+    PyObject *l, *p, *c;
+    if (!PyArg_ParseTuple(args, "OOO", &l, &p, &c)) return nullptr;
+    Py_INCREF(l); Py_INCREF(p); Py_INCREF(c);
+    g_load = l; g_ptr = p; g_cdata = c;
     Py_RETURN_NONE;
 }
 

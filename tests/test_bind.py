@@ -27,6 +27,21 @@ def test_refusals():
     assert bx.ix_gdn_decode(cfg, 1, *[None] * 8, s=0) == bx.HIP_ERROR_INVALID_VALUE
 
 
+def test_descriptions_of_other_types():
+    """A program's own ctypes mirror of the C structures is read like the package's."""
+    import oracle
+    args = [None] * 8
+    assert type(oracle.Cfg()) is not bx.Cfg
+    assert bx.ix_gdn_decode(oracle.Cfg(), 1, *args, s=0) == bx.HIP_ERROR_INVALID_VALUE
+
+    class Gate(ctypes.Structure):
+        _fields_ = bx.OutGate._fields_
+
+    assert bx.ix_gdn_decode_gated(bx.make_cfg(), 1, *args, gate=Gate(), s=0) == bx.HIP_ERROR_INVALID_VALUE
+    with pytest.raises(TypeError):
+        bx.ix_gdn_decode(ctypes.c_int(1), 1, *args, s=0)
+
+
 @pytest.mark.gpu
 def test_streams_and_tensors():
     x = torch.randn(6, 128, device="cuda")
