@@ -10,6 +10,7 @@
 #include "gdn_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace ixg {
 namespace {
@@ -53,6 +54,53 @@ gemv_wave_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
     const int lane = threadIdx.x & (kWave - 1);
     const float r = wave_sum(row_partial(x, w + o * n_in, n_in, lane, kWave, vec));
     if (lane == 0) y[o] = r;
+}
+
+// The same partial (steps in the same order) with the loads of up to 4 steps issued before the first is
+// used: where few waves share a CU, row_partial's steps wait for memory one after the other, 0.6 us
+// each. Rows of n8 16-byte chunks. Batches of 2 alone: 4096 values, 1024 + 1024 rows 5.0 against 4.5 us; of 8 with
+// single steps behind: 2560 values 5.0 against 4.0.
+__device__ __forceinline__ float row_partial_ahead(const uint16_t* __restrict__ x, const uint16_t* __restrict__ row,
+                                                   int n8, int lane) {
+    const u32x4* wv = reinterpret_cast<const u32x4*>(row);
+    const u32x4* xv = reinterpret_cast<const u32x4*>(x);
+    float acc = 0.0f;
+    int i = lane;
+    auto steps = [&](auto count) {                           // count steps of this lane from i on
+        constexpr int N = decltype(count)::value;
+        u32x4 w[N], v[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            w[u] = __builtin_nontemporal_load(wv + i + u * kWave);
+            v[u] = xv[i + u * kWave];
+        }
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                acc = fmaf(bf_lo(v[u][e]), bf_lo(w[u][e]), acc);
+                acc = fmaf(bf_hi(v[u][e]), bf_hi(w[u][e]), acc);
+            }
+        i += N * kWave;
+    };
+    while (i + 3 * kWave < n8) steps(std::integral_constant<int, 4>{});
+    if (i + kWave < n8) steps(std::integral_constant<int, 2>{});
+    if (i < n8) steps(std::integral_constant<int, 1>{});
+    return acc;
+}
+
+// One or two weight matrices against one x, their rows numbered through, one wave per row: bound by
+// the memory's latency until the rows fill the CUs (few_rows).
+__global__ void __launch_bounds__(kGemvThreads)
+gemv_rows_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w1, float* __restrict__ y1, int n_out1,
+                 const uint16_t* __restrict__ w2, float* __restrict__ y2, int n_out2, int n_in) {
+    int o = blockIdx.x * kRowsPerBlock + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int lane = threadIdx.x & (kWave - 1);
+    if (o >= n_out1 + n_out2) return;
+    const bool second = o >= n_out1;
+    if (second) o -= n_out1;
+    const float r = wave_sum(row_partial_ahead(x, (second ? w2 : w1) + (size_t)o * n_in, n_in >> 3, lane));
+    if (lane == 0) (second ? y2 : y1)[o] = r;
 }
 
 // Two weight matrices against one x; row o of each with the same code as gemv_wave_kernel.
@@ -217,6 +265,29 @@ inline bool vec_rows(const uint16_t* x, const uint16_t* w, long long n_in) {
 }
 inline unsigned row_blocks(long long n_out) { return (unsigned)((n_out + kRowsPerBlock - 1) / kRowsPerBlock); }
 
+// gemv_rows_kernel while the rows are all on the GPU at once (8,192 waves fill MI355X), or 4,096 rows of a
+// single matrix: us with the kernels below -> with it,
+//   pair   1024 values, 1024 + 1024 rows 4.0 -> 2.7;  4096 + 4096 5.1 -> 4.5
+//          4096 values,   64 +   64 rows 9.5 -> 3.1;  1024 + 1024 10.7 -> 4.5;  4096 + 4096 13.5 -> 11.3
+//   single 4096 values, 1024 rows 6.1 -> 3.7;  4096 rows 8.0 -> 7.2;  512 values, 2048 rows 2.33 -> 2.37
+// Beyond, a CU's waves hide the latency by themselves, and a row of each matrix on one wave needs
+// fewer waves: 512 values, 8192 + 4096 rows 3.9 against 4.5, 2560 values 11.3 in both (5.6 TB/s); single, 2560
+// values, 6144 rows 6.9 in both. The lines are counts of rows alone, so that they do not move with a row's length.
+constexpr long long kFewRows = 8192, kFewSingle = 4096;
+inline bool few_rows(const uint16_t* x, const uint16_t* w1, long long n1, const uint16_t* w2, long long n2, long long n_in) {
+    if (n1 > kFewRows || n2 > kFewRows || n_in > 1 << 24) return false;       // 32-bit indices
+    if ((n1 > 0 && !vec_rows(x, w1, n_in)) || (n2 > 0 && !vec_rows(x, w2, n_in))) return false;
+    n1 = std::max(n1, 0LL), n2 = std::max(n2, 0LL);
+    return n1 + n2 <= (n1 > 0 && n2 > 0 ? kFewRows : kFewSingle);
+}
+
+inline void launch_rows(const uint16_t* x, const uint16_t* w1, float* y1, long long n_out1, const uint16_t* w2, float* y2,
+                        long long n_out2, long long n_in, hipStream_t s) {
+    const int n1 = (int)std::max(n_out1, 0LL), n2 = (int)std::max(n_out2, 0LL);
+    hipLaunchKernelGGL(gemv_rows_kernel, dim3(row_blocks(n1 + n2)), dim3(kGemvThreads), 0, s, x, w1, y1, n1, w2, y2, n2,
+                       (int)n_in);
+}
+
 // The LDS kernel from 1024 rows (512 rows: 2.1 against 2.0 us with one column) while 8 columns'
 // blocks fit 64 KiB (n_in <= 7264), two workgroups per CU (one: 9.6 against 8.1 us with 8 columns of 4096 ->
 // 6144, four: 9.3). The choice depends on the matrix alone, so that a column's result does not
@@ -255,6 +326,10 @@ extern "C" hipError_t ix_bf16_gemv(const uint16_t* x, const uint16_t* w, float* 
                                    hipStream_t s) {
     if (n_in <= 0 || n_out <= 0) return hipErrorInvalidValue;
     if ((n_out + kRowsPerBlock - 1) / kRowsPerBlock > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (few_rows(x, w, n_out, nullptr, 0, n_in)) {
+        launch_rows(x, w, y, n_out, nullptr, nullptr, 0, n_in, s);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(gemv_wave_kernel, dim3(row_blocks(n_out)), dim3(kGemvThreads), 0, s, x, w, y, n_in, n_out,
                        vec_rows(x, w, n_in));
     return hipGetLastError();
@@ -266,6 +341,10 @@ extern "C" hipError_t ix_bf16_gemv_pair(const uint16_t* x, const uint16_t* w1, f
     if (n_in <= 0 || (n_out1 <= 0 && n_out2 <= 0)) return hipErrorInvalidValue;
     const long long n_out = n_out1 > n_out2 ? n_out1 : n_out2;
     if ((n_out + kRowsPerBlock - 1) / kRowsPerBlock > 0x7fffffffLL) return hipErrorInvalidValue;
+    if (few_rows(x, w1, n_out1, w2, n_out2, n_in)) {
+        launch_rows(x, w1, y1, n_out1, w2, y2, n_out2, n_in, s);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(gemv_pair_kernel, dim3(row_blocks(n_out)), dim3(kGemvThreads), 0, s, x, w1, y1, n_out1,
                        vec_rows(x, w1, n_in), w2, y2, n_out2, vec_rows(x, w2, n_in), n_in);
     return hipGetLastError();
