@@ -156,7 +156,8 @@ __device__ __forceinline__ float bf16_half(uint32_t word, int half) {
     return __uint_as_float(half ? (word & 0xffff0000u) : (word << 16));
 }
 
-template <int DC, bool SILU>
+// THRIFTY: sigmoid_r instead of sigmoid_f.
+template <int DC, bool SILU, bool THRIFTY = false>
 __device__ __forceinline__ void conv_run(ConvIn<DC> in, float (&y0)[kConvTok], float (&y1)[kConvTok]) {
     // Pin the words here: the compiler would otherwise hoist their unpacking up to the loads,
     // which then wait for the data right after issue.
@@ -182,7 +183,10 @@ __device__ __forceinline__ void conv_run(ConvIn<DC> in, float (&y0)[kConvTok], f
         for (int i = 0; i < DC - 1; ++i) { a0 = fmaf(h0[i], w0[i], a0); a1 = fmaf(h1[i], w1[i], a1); }
         a0 = fmaf(x0, w0[DC - 1], a0);
         a1 = fmaf(x1, w1[DC - 1], a1);
-        if constexpr (SILU) { a0 = silu_f(a0); a1 = silu_f(a1); }
+        if constexpr (SILU) {
+            a0 = a0 * (THRIFTY ? sigmoid_r(a0) : sigmoid_f(a0));
+            a1 = a1 * (THRIFTY ? sigmoid_r(a1) : sigmoid_f(a1));
+        }
         y0[t] = a0;
         y1[t] = a1;
 #pragma unroll

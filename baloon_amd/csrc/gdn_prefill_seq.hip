@@ -365,7 +365,7 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
                 const int c2 = 2 * lane, cj = 16 * (4 * (c2 >> 5) + ((c2 >> 2) & 3)), ce = 2 * (4 * ((c2 >> 4) & 1) + (c2 & 3));
                 const int nt = min(max(len - tb, 0), kConvTok);
                 float y0[kConvTok], y1[kConvTok];
-                conv_run<DC, SILU>(in, y0, y1);
+                conv_run<DC, SILU, true>(in, y0, y1);
                 float ss[kConvTok];
 #pragma unroll
                 for (int t = 0; t < kConvTok; ++t) ss[t] = fmaf(y0[t], y0[t], y1[t] * y1[t]);
@@ -592,7 +592,7 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
                             float acc = 0.0f;
 #pragma unroll
                             for (int i = 0; i < DC; ++i) acc = fmaf(xv[e + i], bf16_half(cw[n][i >> 1], i & 1), acc);
-                            if constexpr (SILU) acc = silu_f(acc);
+                            if constexpr (SILU) acc = acc * sigmoid_r(acc);
                             acc = tr + e < len ? acc : 0.0f;
                             W[n][mt][e] = bt[e] * fmaf(-gm[e], W[n][mt][e], acc);
                         }

@@ -73,6 +73,14 @@ def state_from_dev(t) -> np.ndarray:
     return np.ascontiguousarray(np.swapaxes(host(t), -1, -2))
 
 
+def tabled_chunks(ws, n_seq) -> int:
+    """Chunks that the last ix_gdn_prefill of n_seq > 1 sequences on workspace ws (uint8) sent through
+    the windows; the sequences of the others ran one workgroup per sequence. Entry n_seq of the plan's
+    second table (the clamped token offsets before it; both n_seq + 1 int32, 256-byte aligned)."""
+    at = (4 * (n_seq + 1) + 255) // 256 * 256 + 4 * n_seq
+    return int(ws[at:at + 4].cpu().numpy().view(np.int32)[0])
+
+
 def bf16_excess_err(got_bits: np.ndarray, ref_f64: np.ndarray) -> float:
     """max(|bf16 - ref| - half a bf16 ulp): the error beyond bf16's own rounding."""
     ref = np.asarray(ref_f64, dtype=np.float64)
@@ -100,4 +108,4 @@ def bf16_ulp_diff(got_bits: np.ndarray, ref_f64: np.ndarray) -> int:
 
 
 __all__ = ["oracle", "bf16", "inputs", "dev", "host", "state_to_dev", "state_from_dev", "bf16_ulp_diff", "bf16_excess_err",
-           "extreme_gates", "extreme_params", "NT", "TOL_O_ABS", "TOL_STATE_REL"]
+           "extreme_gates", "extreme_params", "tabled_chunks", "NT", "TOL_O_ABS", "TOL_STATE_REL"]
