@@ -274,13 +274,13 @@ __device__ __forceinline__ void out_gate_head(const OutGate& g, size_t row, floa
 __device__ __forceinline__ v4f gate_row4(const OutGate& g, const v4f& o, const v4f& nrm, const uint2& z) {
     float sq = fmaf(o[0], o[0], fmaf(o[1], o[1], fmaf(o[2], o[2], o[3] * o[3])));
     __asm__("" : "+v"(sq));                                  // no part of it fused into the sums
-    const float inv = rsqrtf(fmaf(pair_sum16(row_sum16(sq)), 1.0f / kD, g.eps));
+    const float inv = 1.0f / sqrtf(fmaf(pair_sum16(row_sum16(sq)), 1.0f / kD, g.eps));
     const float zf[4] = {__uint_as_float(z.x << 16), __uint_as_float(z.x & 0xffff0000u), __uint_as_float(z.y << 16),
                          __uint_as_float(z.y & 0xffff0000u)};
     v4f y;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float v = o[e] * inv * nrm[e] * sigmoid_fast(zf[e]);
+        float v = o[e] * inv * nrm[e] * sigmoid_r(zf[e]);
         __asm__("" : "+v"(v));                               // nor this product into a caller's sum
         y[e] = v;
     }

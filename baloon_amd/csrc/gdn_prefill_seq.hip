@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
             for (int mt = 0; mt < 8; ++mt) S[n][mt] = *reinterpret_cast<const v4*>(sl + n * 16 * kD + 16 * mt);
     }
 
-    const int qkch = isk ? k_channel(L, src, 2 * lane0) : q_channel(L, src, 2 * lane0);
+    const int qkch0 = isk ? k_channel(L, src, 0) : q_channel(L, src, 0);
     uint32_t cw[NT][(DC + 1) / 2];                           // conv weights of the lane's v channels, bf16 pairs
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
@@ -239,7 +239,6 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
         for (int i = 0; i < (DC + 1) / 2; ++i)
             cw[n][i] = wp[2 * i] | (2 * i + 1 < DC ? (uint32_t)wp[2 * i + 1] << 16 : 0u);
     }
-    const float A_log = L.A_log[h], dt_bias = L.dt_bias[h];
 
     ChunkGeo g;
     g.s = s;
@@ -250,28 +249,25 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
         g.pos0 = t0 - lo;
     };
     ConvIn<DC> in;
-    uint16_t ra = 0, rb = 0;
-    auto load_gates = [&](const PrefillParams& p) {
-        if (scans) {
-            const size_t ab = (size_t)(g.t0 + min(lane0, g.len - 1)) * p.L.h_v + h;
-            ra = p.a[ab];
-            rb = p.b[ab];
-        }
-    };
     // The outputs of the chunk at t0 from LDS: a row per half wave, 4 columns per lane; wave w of 4-7
     // takes rows 16 (w - 4) .. + 15 of every head. A row's 16-column groups are XOR-swizzled by its
     // row quad.
-    constexpr int R = 8;                                     // two rows at a time
+    constexpr int R = 4;                                     // of 8 pairs of rows, two groups
     auto head_of = [&](const Layer& L, int e) { return mapped_head(L, src, min(m0 + e, nmap - 1)); };
     auto out_at = [&](int e, int row, int col) {
         return (lds_f32*)(ld + LdsOf::kO + e * kOBytes) + row * kD + (col ^ (16 * ((row >> 2) & 3)));
     };
-    auto load_z = [&](const SeqArgs& again, int e, int t0, int len, int lane, int i) {
-        return *reinterpret_cast<const uint2*>(
-            again.gate.z + ((size_t)t0 * again.p.L.h_v + head_of(again.p.L, e)) * kD +
-            ((uint32_t)min(16 * (w - 4) + (lane >> 5) + 2 * i, len - 1) * again.p.L.h_v * kD + 4 * (lane & 31)));
+    auto load_z = [&](int e, int i0, int t0, int len, int lane, uint2 (&z)[R]) {
+        const SeqArgs again = args_again();
+        const int hv = again.p.L.h_v;
+        const uint16_t* zb = again.gate.z + ((size_t)t0 * hv + head_of(again.p.L, e)) * kD;
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            z[i] = *reinterpret_cast<const uint2*>(
+                zb + ((uint32_t)min(16 * (w - 4) + (lane >> 5) + 2 * (i0 + i), len - 1) * hv * kD + 4 * (lane & 31)));
     };
-    auto out_rows = [&](int e, const uint2* z, int t0, int len, int lane) {
+    // Row pairs i0 .. i0 + R - 1 of head e.
+    auto out_rows = [&](int e, int i0, const uint2 (&z)[R], int t0, int len, int lane) {
         const SeqArgs again = args_again();
         const PrefillParams& p = again.p;
         const OutGate& gate = again.gate;
@@ -284,42 +280,35 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
             return __builtin_amdgcn_make_buffer_rsrc(static_cast<char*>(out) + base * bytes, 0,
                                                      live ? (int)(((uint32_t)(len - 1) * ostep + kD) * bytes) : 0, 0x00020000);
         };
-        const int r0 = 16 * (w - 4) + (lane >> 5), oc = 4 * (lane & 31);
+        const int r0 = 16 * (w - 4) + (lane >> 5) + 2 * i0, oc = 4 * (lane & 31);
         const uint32_t at = (uint32_t)r0 * ostep + oc;
         v4 nrm;
         if constexpr (GATED) nrm = *reinterpret_cast<const v4*>(gate.nrm + oc);
+        v4 o[R];
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            constexpr int H = R / 2;
-            const int i0 = half * H;
-            v4 o[H];
+        for (int i = 0; i < R; ++i) o[i] = *(const lds_v4*)out_at(e, r0 + 2 * i, oc);
+        auto store32 = [&](float* out) {
+            const auto b = rows_of(out, 4);
 #pragma unroll
-            for (int i = 0; i < H; ++i) o[i] = *(const lds_v4*)out_at(e, r0 + 2 * (i0 + i), oc);
-            auto store32 = [&](float* out) {
-                const auto b = rows_of(out, 4);
+            for (int i = 0; i < R; ++i)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4x, o[i]), b, (at + 2 * i * ostep) * 4, 0, 0);
+        };
+        auto store16 = [&](uint16_t* out) {
+            const auto b = rows_of(out, 2);
 #pragma unroll
-                for (int i = 0; i < H; ++i)
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4x, o[i]), b, (at + 2 * (i0 + i) * ostep) * 4, 0, 0);
-            };
-            auto store16 = [&](uint16_t* out) {
-                const auto b = rows_of(out, 2);
-#pragma unroll
-                for (int i = 0; i < H; ++i)
-                    __builtin_amdgcn_raw_buffer_store_b64(u2x{pack_bf16x2(o[i][0], o[i][1]), pack_bf16x2(o[i][2], o[i][3])}, b,
-                                                          (at + 2 * (i0 + i) * ostep) * 2, 0, 0);
-            };
-            if (p.o) store32(p.o);
-            if (p.o_bf16) store16(p.o_bf16);
-            if constexpr (GATED) {
-#pragma unroll
-                for (int i = 0; i < H; ++i) o[i] = gate_row4(gate, o[i], nrm, z[i0 + i]);
-                if (gate.y) store32(gate.y);
-                if (gate.y_bf16) store16(gate.y_bf16);
-            }
-        }
+            for (int i = 0; i < R; ++i)
+                __builtin_amdgcn_raw_buffer_store_b64(u2x{pack_bf16x2(o[i][0], o[i][1]), pack_bf16x2(o[i][2], o[i][3])}, b,
+                                                      (at + 2 * i * ostep) * 2, 0, 0);
+        };
+        if (p.o) store32(p.o);
+        if (p.o_bf16) store16(p.o_bf16);
         if constexpr (GATED) {
-            // q8_1 blocks from the same values, formed again: kept apart and rolled up, their divisions
-            // would otherwise be most of the loop's code.
+#pragma unroll
+            for (int i = 0; i < R; ++i) o[i] = gate_row4(gate, o[i], nrm, z[i]);
+            if (gate.y) store32(gate.y);
+            if (gate.y_bf16) store16(gate.y_bf16);
+            // q8_1 blocks from the same values, formed for themselves: kept apart and rolled up, their
+            // divisions would otherwise be most of the loop's code.
             if (gate.y_q8_1) {
 #pragma clang loop unroll(disable)
                 for (int i = 0; i < R; ++i) {
@@ -334,10 +323,9 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
     };
 
     geo(lo);
-    row_load_first<DC>(p, g, qkch, tb, in);
-    load_gates(p);
+    row_load_first<DC>(p, g, qkch0 + 2 * lane0, tb, in);
 #pragma unroll
-    for (int i = 0; i < kConvTok / 2; ++i) row_load_pair<DC>(p, g, qkch, tb, i, in);
+    for (int i = 0; i < kConvTok / 2; ++i) row_load_pair<DC>(p, g, qkch0 + 2 * lane0, tb, i, in);
     VIn<NT> vin;
     const int vch = v_channel(L, h, col0);
 #pragma unroll
@@ -358,7 +346,17 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
         const bool main = t0 < hi;                           // false once more, for the last outputs
         u2x uh[NH][2] = {}, ul[NH][2] = {};
         if (main) {
-            // 1. q and k rows
+            // 1. q and k rows; the gate inputs of the scanning waves, loaded ahead of them (lane = token)
+            uint16_t ra = 0, rb = 0;
+            float A_log = 0.0f, dt_bias = 0.0f;
+            if (scans) {
+                const SeqArgs again = args_again();
+                const size_t ab = (size_t)(t0 + min(lane, len - 1)) * again.p.L.h_v + h;
+                ra = again.p.a[ab];
+                rb = again.p.b[ab];
+                A_log = again.p.L.A_log[h];
+                dt_bias = again.p.L.dt_bias[h];
+            }
             {
                 // Channel pair (2 l, 2 l + 1) of a plane row: channel 32 b + 16 u + 4 a + e sits in
                 // chunk 4 b + a at entry 4 u + e.
@@ -521,16 +519,14 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
         phase();
         if (w >= 4 && t0 > lo) {
             const int tp = t0 - kChunk, lp = min(kChunk, hi - tp);
-            uint2 z[NH][R];                                  // the gate's inputs
-            if constexpr (GATED) {
-                const SeqArgs again = args_again();
+            uint2 z[2][R];                                   // the gate's inputs of a group, the next one's ahead
+            if constexpr (GATED) load_z(0, 0, tp, lp, lane, z[0]);
 #pragma unroll
-                for (int e = 0; e < NH; ++e)
-#pragma unroll
-                    for (int i = 0; i < R; ++i) z[e][i] = load_z(again, e, tp, lp, lane, i);
+            for (int i = 0; i < 2 * NH; ++i) {
+                if constexpr (GATED)
+                    if (i + 1 < 2 * NH) load_z((i + 1) >> 1, R * ((i + 1) & 1), tp, lp, lane, z[(i + 1) & 1]);
+                out_rows(i >> 1, R * (i & 1), z[i & 1], tp, lp, lane);
             }
-#pragma unroll
-            for (int e = 0; e < NH; ++e) out_rows(e, z[e], tp, lp, lane);
         }
         if (!main) break;
         lds_barrier();
@@ -676,7 +672,7 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
             phase();
             if (t0 + kChunk < hi) geo(t0 + kChunk);
             const SeqArgs again = args_again();
-            row_load_first<DC>(again.p, g, qkch, tb, in);
+            row_load_first<DC>(again.p, g, qkch0 + 2 * lane, tb, in);
             const float gam = dec_of(hd, 2)[kChunk - 1];
             bf8 f[2][4];                                     // K^T of a row tile, the next one's read ahead
             auto operands = [&](int mt, bf8 (&x)[4]) {
@@ -693,13 +689,12 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
                 const bf8(&x)[4] = f[mt & 1];
                 mfma_tiles<NT>(x[0], x[1], eh[0], el[0], S, mt);
                 mfma_tiles<NT>(x[2], x[3], eh[1], el[1], S, mt);
-                row_load_pair<DC>(again.p, g, qkch, tb, mt, in);
+                row_load_pair<DC>(again.p, g, qkch0 + 2 * lane, tb, mt, in);
                 v_load<NT>(again.p, g, hi - lo - 1, vch, lane, mt, vin);
                 if (mt == 7) v_load<NT>(again.p, g, hi - lo - 1, vch, lane, 8, vin);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        load_gates(args_again().p);
         lds_barrier();                                       // keys, A, T and M read for the last time
     }
     if (m0 + hd >= nmap) return;

@@ -158,7 +158,4 @@ __device__ __forceinline__ float sigmoid_r(float x) {
     return t >= 128.0f ? 0.0f : v * kScale;                  // e infinite
 }
 
-// sigmoid on the hardware exp and reciprocal (1 ulp each; relative error below 1e-6 for |x| < 10).
-__device__ __forceinline__ float sigmoid_fast(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
-
 }  // namespace ixg

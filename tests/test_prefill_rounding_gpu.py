@@ -90,3 +90,19 @@ def test_silu(route):
     s, o, _ = prefill(route, cfg, [1] * n, x, full(-100.0), full(-200.0),
                       np.broadcast_to(np.eye(128, dtype=np.float32), (n, 8, 128, 128)))
     assert differing(o[..., 1:], k[:, src, 1:]) <= DIFFER
+
+
+@pytest.mark.parametrize("route", ["seq", "windows"])
+def test_output_gate(route):
+    """y from the call's own fp32 o: the sum of 128 squares (at most 9 roundings, halved by the root), its
+    scaling, root and reciprocal, three products and the sigmoid (an ulp), each half an ulp."""
+    cfg = bx.make_cfg(h_k=4, h_v=8)
+    rng = np.random.default_rng(3)
+    x, z = rng.standard_normal((N, 16 * 128)), bf16.round_f32(rng.uniform(-80.0, 80.0, (N, 8, 128)))
+    nrm = (1.0 + 0.1 * rng.standard_normal(128)).astype(np.float32)
+    _, o, y = prefill(route, cfg, [1] * N, x, rng.standard_normal((N, 8)), rng.standard_normal((N, 8)),
+                      0.02 * rng.standard_normal((N, 8, 128, 128)), (z, nrm))
+    o = o.astype(np.float64)
+    want = o / np.sqrt((o * o).mean(-1, keepdims=True) + 1e-6) * nrm / (1.0 + np.exp(-z.astype(np.float64)))
+    err = float(np.max(np.abs(y / want - 1.0)))
+    assert err <= (4.5 + 1.0 + 3 * 1.0 + 1.5 + 2.0) * 2.0 ** -24, err
