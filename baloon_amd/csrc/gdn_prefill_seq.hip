@@ -388,8 +388,8 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
                 const float last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lg), kChunk - 1));
                 dec_of(hd, 0)[lane] = lg;
                 dec_of(hd, 1)[lane] = ok ? sigmoid_f(bf16_to_f32(rb)) : 0.0f;
-                dec_of(hd, 2)[lane] = __expf(lg);
-                dec_of(hd, 3)[lane] = __expf(last - lg);
+                dec_of(hd, 2)[lane] = expf(lg);
+                dec_of(hd, 3)[lane] = expf(last - lg);
             }
             lds_barrier();
 

@@ -93,6 +93,29 @@ def test_silu(route):
 
 
 @pytest.mark.parametrize("route", ["seq", "windows"])
+def test_decay(route):
+    """Whole gate logits above softplus's threshold: the log decay is minus the logit, exactly."""
+    cfg = bx.make_cfg(h_k=4, h_v=8)
+    rng = np.random.default_rng(2)
+    a = (21 + np.arange(N * 8) % 40).reshape(N, 8).astype(np.float32)
+    x = np.zeros((N, 16, 128), np.float32)
+    x[:, :8, 0] = 50.0                                         # q = k = the first unit vector
+    x[:, 8:] = bf16.round_f32(rng.standard_normal((N, 8, 128)))
+    state = bf16.round_f32(rng.standard_normal((N, 8, 128, 128)))
+    # beta = 0: S' = exp(-a) S, to the exponential's and the product's rounding; o = its row 0, times
+    # q's factor (a square root and two products) twice rounded.
+    s, o, _ = prefill(route, cfg, [1] * N, x.reshape(N, -1), a, np.full((N, 8), -200.0), state)
+    want = np.exp(-a.astype(np.float64))[:, :, None, None] * state
+    assert float(np.max(np.abs(s / want - 1.0))) <= 1.5 * 2.0 ** -23
+    assert float(np.max(np.abs(o / want[:, :, 0] - 1.0))) <= 4.5 * 2.0 ** -23
+    # Two tokens, S = 0, beta = 1 and then 0: S' = exp(-a_1) k v_0^T.
+    two = lambda u, v: np.stack([u, v], 1).reshape(2 * N, -1)  # noqa: E731
+    s, _, _ = prefill(route, cfg, [2] * N, two(x.reshape(N, -1), x.reshape(N, -1)), two(a, a),
+                      two(np.full((N, 8), 30.0), np.full((N, 8), -200.0)), np.zeros_like(state))
+    assert differing(s[:, :, 0], split(np.exp(-a.astype(np.float64))[..., None] * x[:, 8:])) <= DIFFER
+
+
+@pytest.mark.parametrize("route", ["seq", "windows"])
 def test_output_gate(route):
     """y from the call's own fp32 o: the sum of 128 squares (at most 9 roundings, halved by the root), its
     scaling, root and reciprocal, three products and the sigmoid (an ulp), each half an ulp."""
