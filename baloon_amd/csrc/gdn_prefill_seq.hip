@@ -283,7 +283,21 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
         const int r0 = 16 * (w - 4) + (lane >> 5) + 2 * i0, oc = 4 * (lane & 31);
         const uint32_t at = (uint32_t)r0 * ostep + oc;
         v4 nrm;
-        if constexpr (GATED) nrm = *reinterpret_cast<const v4*>(gate.nrm + oc);
+        if constexpr (GATED) {
+            nrm = *reinterpret_cast<const v4*>(gate.nrm + oc);
+            // q8_1 blocks from the same values, formed for themselves: kept apart and rolled up, their
+            // divisions would otherwise be most of the loop's code. Ahead of the stores: y_bf16 may overwrite z.
+            if (gate.y_q8_1) {
+#pragma clang loop unroll(disable)
+                for (int i = 0; i < R; ++i) {
+                    const int row = r0 + 2 * i;
+                    const uint32_t ra = (uint32_t)min(row, len - 1) * ostep + oc;
+                    const v4 v = *(const lds_v4*)out_at(e, row, oc);
+                    const v4 y = gate_row4(gate, v, nrm, *reinterpret_cast<const uint2*>(gate.z + base + ra));
+                    q81_store4(y, lane, live && row < len ? gate.y_q8_1 + (base + ra) / 32 * kQ81Bytes : nullptr);
+                }
+            }
+        }
         v4 o[R];
 #pragma unroll
         for (int i = 0; i < R; ++i) o[i] = *(const lds_v4*)out_at(e, r0 + 2 * i, oc);
@@ -307,18 +321,6 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
             for (int i = 0; i < R; ++i) o[i] = gate_row4(gate, o[i], nrm, z[i]);
             if (gate.y) store32(gate.y);
             if (gate.y_bf16) store16(gate.y_bf16);
-            // q8_1 blocks from the same values, formed for themselves: kept apart and rolled up, their
-            // divisions would otherwise be most of the loop's code.
-            if (gate.y_q8_1) {
-#pragma clang loop unroll(disable)
-                for (int i = 0; i < R; ++i) {
-                    const int row = r0 + 2 * i;
-                    const uint32_t ra = (uint32_t)min(row, len - 1) * ostep + oc;
-                    const v4 v = *(const lds_v4*)out_at(e, row, oc);
-                    const v4 y = gate_row4(gate, v, nrm, *reinterpret_cast<const uint2*>(gate.z + base + ra));
-                    q81_store4(y, lane, live && row < len ? gate.y_q8_1 + (base + ra) / 32 * kQ81Bytes : nullptr);
-                }
-            }
         }
     };
 

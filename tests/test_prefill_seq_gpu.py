@@ -11,7 +11,7 @@ import pytest
 import baloon_amd as bx
 import oracle
 from oracle import bf16, inputs
-from tests.common import NT, TOL_O_ABS, TOL_STATE_REL, dev, host, state_from_dev, state_to_dev
+from tests.common import NT, TOL_O_ABS, TOL_STATE_REL, dev, host, state_from_dev, state_to_dev, tabled_chunks
 
 pytestmark = pytest.mark.gpu
 
@@ -79,3 +79,35 @@ def test_many_sequences(kw, n, longest):
     np.testing.assert_array_equal(yb, bf16.from_f32(y))
     for a, b in zip((gcs, gs, y, yb), run(cfg, cu, tok, p, st, g, window=2)):
         np.testing.assert_array_equal(a, b)                    # whatever the workspace
+
+
+def chunks(lens):
+    return sum((v + 63) // 64 for v in lens)
+
+
+@pytest.mark.parametrize("n", [1, 3, 64])
+def test_output_over_the_gate_inputs(n):
+    """y_bf16 may overwrite z, row by row, whatever else is written: on one sequence, in windows, by sequence."""
+    import torch
+    cfg = bx.make_cfg(h_k=4, h_v=8)
+    lens = [1 + (37 * s) % 100 for s in range(n)]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, seed = int(cu[-1]), inputs.seed_for(4) + 78 + n
+    p, tok, st = inputs.layer_params(cfg, seed), inputs.token_inputs(cfg, seed, T), inputs.initial_states(cfg, seed, n)
+    g = inputs.out_gate_inputs(cfg, seed, T)
+    need = bx.ix_gdn_prefill_gated_workspace_size(cfg, n, T)
+
+    def call(over):
+        z, ws = dev(g["z"]), torch.empty(need, dtype=torch.uint8, device="cuda")
+        y, yb = torch.zeros(T, 8, 128, device="cuda"), z if over else torch.zeros_like(z)
+        yq, nrm = torch.zeros(T * 8 * 4 * 36, dtype=torch.uint8, device="cuda"), dev(g["nrm"])
+        assert bx.ix_gdn_prefill_gated(cfg, n, T, dev(cu), dev(tok["x"]), dev(st["conv_state"]), dev(p["w"]), dev(tok["a"]),
+                                       dev(tok["b"]), dev(p["A_log"]), dev(p["dt_bias"]), state_to_dev(st["state"]),
+                                       gate=bx.out_gate(z, nrm, 1e-6, y, yb, yq), workspace=ws,
+                                       workspace_bytes=need) == 0
+        torch.cuda.synchronize()
+        assert n == 1 or tabled_chunks(ws, n) == (0 if n == 64 else chunks(lens))
+        return host(y), host(yb), host(yq)
+
+    for u, v in zip(call(False), call(True)):
+        np.testing.assert_array_equal(u, v)
