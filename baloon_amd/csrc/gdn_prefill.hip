@@ -77,7 +77,7 @@ __device__ int block_inclusive_scan(int v, int* wave_tot) {
 
 __global__ void __launch_bounds__(kPlanThreads) plan_kernel(const PrefillParams p) {
     __shared__ int wave_tot[kPlanThreads / kWave];
-    __shared__ int carry;
+    __shared__ int carry, most;
     __shared__ int hist[kPlanThreads];
     __shared__ unsigned long long best[kPlanThreads / kWave];
     const int tid = threadIdx.x, n = p.n_seq;
@@ -98,20 +98,24 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(const PrefillParams 
     // others, listed longest first, to seq_kernel; `longest` minimises the two parts' time. Thread v
     // prices v: seq_kernel runs its longest sequence's chunks one after the other (cost_seq each)
     // or, if that is more, the GPU's share of all its work (cost_work per chunk); the windows take
-    // cost_win per chunk of the table.
+    // cost_win per chunk of the table. The last thread stands for every length from its own on and
+    // prices the batch's longest.
     int longest = 0;
     if (p.by_seq) {
         hist[tid] = 0;
+        if (tid == 0) most = 0;
         __syncthreads();
         for (int s = tid; s < n; s += kPlanThreads) {
             const int c = chunks_of(s);
             atomicAdd(&hist[min(c, kPlanThreads - 1)], c);
+            if (c >= kPlanThreads) atomicMax(&most, c);
         }
         __syncthreads();
         const int upto = block_inclusive_scan<false>(hist[tid], wave_tot);   // chunks of lengths <= tid
         if (tid == kPlanThreads - 1) carry = upto;
         __syncthreads();
-        const float cost = p.cost_win * (float)(carry - upto) + fmaxf(p.cost_seq * (float)tid, p.cost_work * (float)upto);
+        const int walk = tid < kPlanThreads - 1 ? tid : max(tid, most);
+        const float cost = p.cost_win * (float)(carry - upto) + fmaxf(p.cost_seq * (float)walk, p.cost_work * (float)upto);
         // the least cost, the shortest length on a tie: (cost, length) as one 64-bit key
         unsigned long long key = ((unsigned long long)__float_as_uint(cost) << 32) | (unsigned)tid;
 #pragma unroll

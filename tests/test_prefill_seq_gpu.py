@@ -111,3 +111,23 @@ def test_output_over_the_gate_inputs(n):
 
     for u, v in zip(call(False), call(True)):
         np.testing.assert_array_equal(u, v)
+
+
+def test_plan_prices_long_sequences():
+    """A walk is as long as its longest sequence, also past the lengths the plan tells apart: one of
+    3,000 chunks among short ones goes through the windows (30 ms against 55 in a workgroup of its own), the
+    others do not. (Zero inputs: the plan sees the lengths alone.)"""
+    import torch
+    cfg = bx.make_cfg(h_k=16, h_v=96)
+    lens = [3000 * 64, 10, 70, 0, 130]
+    n, T, C = len(lens), sum(lens), cfg.channels
+    bf = dict(dtype=torch.bfloat16, device="cuda")
+    x, a = torch.zeros(T, C, **bf), torch.zeros(T, 96, **bf)
+    cu = dev(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+    need = bx.ix_gdn_prefill_workspace_size(cfg, n, T)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    assert bx.ix_gdn_prefill(cfg, n, T, cu, x, torch.zeros(n, C, 3, **bf), torch.zeros(C, 4, **bf), a, a,
+                             torch.zeros(96, device="cuda"), torch.zeros(96, device="cuda"),
+                             torch.zeros(n, 96, 128, 128, device="cuda"), workspace=ws, workspace_bytes=need) == 0
+    torch.cuda.synchronize()
+    assert tabled_chunks(ws, n) == 3000
