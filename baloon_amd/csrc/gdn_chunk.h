@@ -88,7 +88,7 @@ struct PrefillParams {
     int cb, W;                  // the window: chunks cb .. cb + W - 1
     int G;                      // chain workgroups per (v head, strip) in a window (1 for n_seq == 1)
     int by_seq;                 // sequences up to a length that the plan chooses go to seq_kernel
-    float cost_seq, cost_work, cost_win;   // its prices (us per chunk)
+    float cost_start, cost_seq, cost_work, cost_win, cost_chain;   // its prices (us; the first once, the others per chunk)
     int o_win;                  // o holds the window's chunks only, 64 rows each
 };
 

@@ -96,10 +96,10 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(const PrefillParams 
     }
     // With by_seq, the sequences of more than `longest` chunks go through the chunk table and the
     // others, listed longest first, to seq_kernel; `longest` minimises the two parts' time. Thread v
-    // prices v: seq_kernel runs its longest sequence's chunks one after the other (cost_seq each)
-    // or, if that is more, the GPU's share of all its work (cost_work per chunk); the windows take
-    // cost_win per chunk of the table. The last thread stands for every length from its own on and
-    // prices the batch's longest.
+    // prices v: seq_kernel starts (cost_start) and runs its longest sequence's chunks one after the other
+    // (cost_seq each) or, if that is more, the GPU's share of all its work (cost_work per chunk); the windows take
+    // cost_win per chunk of the table and, in the chain, cost_chain per chunk of its longest group. The
+    // last thread stands for every length from its own on and prices the batch's longest.
     int longest = 0;
     if (p.by_seq) {
         hist[tid] = 0;
@@ -108,14 +108,17 @@ __global__ void __launch_bounds__(kPlanThreads) plan_kernel(const PrefillParams 
         for (int s = tid; s < n; s += kPlanThreads) {
             const int c = chunks_of(s);
             atomicAdd(&hist[min(c, kPlanThreads - 1)], c);
-            if (c >= kPlanThreads) atomicMax(&most, c);
+            atomicMax(&most, c);
         }
         __syncthreads();
         const int upto = block_inclusive_scan<false>(hist[tid], wave_tot);   // chunks of lengths <= tid
         if (tid == kPlanThreads - 1) carry = upto;
         __syncthreads();
         const int walk = tid < kPlanThreads - 1 ? tid : max(tid, most);
-        const float cost = p.cost_win * (float)(carry - upto) + fmaxf(p.cost_seq * (float)walk, p.cost_work * (float)upto);
+        const int rest = carry - upto;
+        const float chain = rest ? p.cost_chain * fmaxf((float)rest / (float)p.G, (float)most) : 0.0f;
+        const float cost = p.cost_win * (float)rest + chain +
+                           (upto ? p.cost_start + fmaxf(p.cost_seq * (float)walk, p.cost_work * (float)upto) : 0.0f);
         // the least cost, the shortest length on a tie: (cost, length) as one 64-bit key
         unsigned long long key = ((unsigned long long)__float_as_uint(cost) << 32) | (unsigned)tid;
 #pragma unroll
@@ -1473,12 +1476,11 @@ static void launch_prefill(const ixg::PrefillParams& p, dim3 tgrid, dim3 cgrid, 
 
 // Whether the batch's sequences may run one workgroup per (sequence, up to two v heads of a q/k
 // head) (gdn_prefill_seq.hip): the pointers allow its vector accesses, the offsets its 32-bit
-// arithmetic, T' of one chunk's space its list of sequences, and there are enough workgroups
-// that batches of even lengths gain: at 12 and 16 sequences of U[1, 2048] tokens 16 q/k and 32 v heads
-// took 579 and 511 us against 662 and 768 us in windows, at 8 605 against 623, at 4 571 against 301; 16
-// and 48 heads (two workgroups per q/k head) 339 against 438 at 6; 8 and 16 heads 574 against 786
-// at 24, 590 against 566 at 16. Which of the sequences then do is decided on the device, from
-// their lengths (plan_kernel).
+// arithmetic, T' of one chunk's space its list of sequences, and there are enough workgroups for a gain.
+// Which of the sequences then do is decided on the device, from their lengths (plan_kernel): with
+// SiLU and output gate, U[1, 2048] tokens, 16 q/k and 32 v heads, 12 sequences take 643 us in windows (741 by
+// sequence), 14 742 us by sequence (757 in windows), 16 753 (877), 32 847 (1,744); plain ones 426 (506), 497 in
+// windows (510), 516 (572), 580 (1,131).
 constexpr long long kSeqWorkgroups = 176;
 static bool by_sequence(const ixg::PrefillParams& p, const ixg::OutGate& g, bool gated) {
     auto on = [](const void* q, uintptr_t a) { return (reinterpret_cast<uintptr_t>(q) & (a - 1)) == 0; };
@@ -1533,13 +1535,25 @@ static hipError_t prefill_impl(const ix_gdn_cfg* cfg, int n_seq, int total_T, co
     const OutGate og = make_out_gate(gate);
     const bool silu = cfg->conv_act == IX_GDN_ACT_SILU;
     p.by_seq = by_sequence(p, og, gate != nullptr);
+    // Chain workgroups: (v head, strip, group), G groups splitting each window's chunks at sequence
+    // starts; one group while the h_v * 8 (head, strip) runs fill every CU.
+    p.G = 1;
+    if (!p.single) p.G = std::max(1, std::min(n_seq, ixg::device_cu_count(s) / (cfg->h_v * kStrips)));
     if (p.by_seq) {
-        // Measured: a chunk of a workgroup's walk 18.3 us with two heads, 12.2 with one (19 and 13 with
-        // the GPU full); in windows 3.3 us per chunk at 32 v heads, more or less in proportion.
-        const float one = cfg->h_v > cfg->h_k ? 18.3f : 12.2f;
-        p.cost_seq = one;
-        p.cost_work = 1.05f * one * (float)seq_workgroups(p.L) / (float)device_cu_count(s);
-        p.cost_win = 3.3f * (float)cfg->h_v / 32.0f;
+        // The plan's prices in us, with SiLU and with the output gate dearer by the vector work of each.
+        // A chunk of a walk with two heads takes 16.5 us, with both 23.7; with one head 11.2 and 15.8. A window's
+        // chunk takes 0.4 (launches and the kernels' latencies, 35 us per 80 chunks), 0.03 per workgroup of
+        // the chunk kernel and 1.5 in the chain, whose groups run side by side (a sequence in one of them) and
+        // whose workgroups past one per CU run in a second round. Fitted to 15 head layouts from 1 and 2 to 16 and 64 heads (0.6 to
+        // 7.2 us per window chunk): within 13% of them, but for 32 and 32 heads (a quarter below).
+        const float silu1 = silu ? 1.0f : 0.0f, gate1 = gate ? 1.0f : 0.0f;
+        const long long wg = seq_workgroups(p.L), cu = device_cu_count(s);
+        const float rounds = (float)(((long long)cfg->h_v * kStrips + cu - 1) / cu);
+        p.cost_start = 15.0f;
+        p.cost_seq = cfg->h_v > cfg->h_k ? 16.5f + 3.0f * silu1 + 4.0f * gate1 : 11.2f + 2.6f * silu1 + 2.0f * gate1;
+        p.cost_work = 1.05f * p.cost_seq * (float)wg / (float)cu;
+        p.cost_win = 0.4f + 0.03f * (float)wg + (float)cfg->h_v * (0.01f * silu1 + 0.03f * gate1);
+        p.cost_chain = 1.5f * rounds;
     }
     if (!p.single) hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, p);
     if (p.by_seq) {
@@ -1548,11 +1562,7 @@ static hipError_t prefill_impl(const ix_gdn_cfg* cfg, int n_seq, int total_T, co
         launch_prefill_seq(q, gate ? &og : nullptr, silu, s);
     }
 
-    // The rest, or everything: chunk kernel and chain per window. Chain workgroups: (v head, strip,
-    // group), G groups splitting each window's chunks at sequence starts; one group while the
-    // h_v * 8 (head, strip) runs fill every CU.
-    p.G = 1;
-    if (!p.single) p.G = std::max(1, std::min(n_seq, ixg::device_cu_count(s) / (cfg->h_v * kStrips)));
+    // The rest, or everything: chunk kernel and chain per window.
     const long long groups = ((long long)p.G * cfg->h_v + 7) / 8;
     const dim3 cgrid((unsigned)(groups * 8 * kStrips)), cblock(kChainWaves * kWave);
     // Windows run in stream order: each chain resumes from the state and conv history the

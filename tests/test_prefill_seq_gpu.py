@@ -5,6 +5,8 @@ Tolerances as in test_prefill_gpu.py (outputs 1e-3 absolute, state max|d|/max|re
 and bf16 rounding exact); y against the norm of the double outputs 1e-4 (test_gated_gpu.py's
 end-to-end bound); q8_1 bytes equal the separate quantiser's.
 """
+import random
+
 import numpy as np
 import pytest
 
@@ -115,11 +117,11 @@ def test_output_over_the_gate_inputs(n):
 
 def test_plan_prices_long_sequences():
     """A walk is as long as its longest sequence, also past the lengths the plan tells apart: one of
-    3,000 chunks among short ones goes through the windows (30 ms against 55 in a workgroup of its own), the
+    3,000 chunks among short ones goes through the windows (19 ms against 50 in a workgroup of its own), the
     others do not. (Zero inputs: the plan sees the lengths alone.)"""
     import torch
     cfg = bx.make_cfg(h_k=16, h_v=96)
-    lens = [3000 * 64, 10, 70, 0, 130]
+    lens = [3000 * 64] + [100] * 40
     n, T, C = len(lens), sum(lens), cfg.channels
     bf = dict(dtype=torch.bfloat16, device="cuda")
     x, a = torch.zeros(T, C, **bf), torch.zeros(T, 96, **bf)
@@ -131,3 +133,26 @@ def test_plan_prices_long_sequences():
                              torch.zeros(n, 96, 128, 128, device="cuda"), workspace=ws, workspace_bytes=need) == 0
     torch.cuda.synchronize()
     assert tabled_chunks(ws, n) == 3000
+
+
+@pytest.mark.parametrize("n,gated,tabled", [(12, False, True), (12, True, True), (32, False, False), (32, True, False)])
+def test_plan_routes(n, gated, tabled):
+    """U[1, 2048] tokens, 16 q/k and 32 v heads: 12 sequences fill too few CUs and are faster in windows, 32 are
+    faster by sequence (measured at by_sequence, gdn_prefill.hip). Zero inputs: the plan sees the lengths alone."""
+    import torch
+    cfg = bx.make_cfg(conv_act=int(gated))
+    rng = random.Random(4)
+    lens = [rng.randint(1, 2048) for _ in range(n)]
+    T, bf = sum(lens), dict(dtype=torch.bfloat16, device="cuda")
+    x, a = torch.zeros(T, cfg.channels, **bf), torch.zeros(T, 32, **bf)
+    z, yb, nrm = torch.zeros(T, 32, 128, **bf), torch.empty(T, 32, 128, **bf), torch.ones(128, device="cuda")
+    need = bx.ix_gdn_prefill_gated_workspace_size(cfg, n, T)
+    ws, zero = torch.empty(need, dtype=torch.uint8, device="cuda"), torch.zeros(32, device="cuda")
+    args = (cfg, n, T, dev(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)), x, torch.zeros(n, cfg.channels, 3, **bf),
+            torch.zeros(cfg.channels, 4, **bf), a, a, zero, zero, torch.zeros(n, 32, 128, 128, device="cuda"))
+    if gated:
+        assert bx.ix_gdn_prefill_gated(*args, gate=bx.out_gate(z, nrm, 1e-6, None, yb), workspace=ws, workspace_bytes=need) == 0
+    else:
+        assert bx.ix_gdn_prefill(*args, o_bf16=yb, workspace=ws, workspace_bytes=need) == 0
+    torch.cuda.synchronize()
+    assert tabled_chunks(ws, n) == (chunks(lens) if tabled else 0)
