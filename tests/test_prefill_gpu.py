@@ -13,7 +13,7 @@ import baloon_amd as bx
 import oracle
 from oracle import bf16, inputs
 from tests.common import (NT, TOL_O_ABS, TOL_STATE_REL, dev, extreme_gates, extreme_params, host, state_from_dev,
-                          state_to_dev)
+                          state_to_dev, tabled_chunks)
 
 pytestmark = pytest.mark.gpu
 
@@ -23,15 +23,19 @@ def _torch():
     return torch
 
 
-def gpu_prefill(cfg, cu, tok, p, st, outputs=("o", "ob"), window=None):
+def gpu_prefill(cfg, cu, tok, p, st, outputs=("o", "ob"), window=None, windows_only=False):
     """Runs ix_gdn_prefill on copies of the states; returns (conv_state, state, o, o_bf16). With
-    window, the workspace holds windows of that many chunks only."""
+    window, the workspace holds windows of that many chunks only. windows_only keeps a batch of many
+    sequences in the windows (an o_bf16 off 8 bytes is not for a workgroup per sequence) and
+    checks that all its chunks went there."""
     torch = _torch()
     cu = np.asarray(cu, np.int32)
     n, T = cu.size - 1, int(tok["x"].shape[0])
     d_cs, d_st = dev(st["conv_state"]), state_to_dev(st["state"])
     o = torch.full((T, cfg.h_v, cfg.d_v), float("nan"), dtype=torch.float32, device="cuda") if "o" in outputs else None
     ob = torch.zeros(T, cfg.h_v, cfg.d_v, dtype=torch.bfloat16, device="cuda") if "ob" in outputs else None
+    if windows_only:
+        ob = torch.zeros(T * cfg.h_v * cfg.d_v + 1, dtype=torch.bfloat16, device="cuda")[1:].view(T, cfg.h_v, cfg.d_v)
     need = (bx.ix_gdn_prefill_workspace_size(cfg, n, T) if window is None
             else bx.ix_gdn_prefill_window_workspace_size(cfg, n, T, window))
     assert need > 0
@@ -40,6 +44,8 @@ def gpu_prefill(cfg, cu, tok, p, st, outputs=("o", "ob"), window=None):
                            dev(p["A_log"]), dev(p["dt_bias"]), d_st, o, ob, ws, need)
     assert rc == 0, rc
     torch.cuda.synchronize()
+    if windows_only:
+        assert tabled_chunks(ws, n) == int(((np.diff(cu) + 63) // 64).sum())
     return (host(d_cs), state_from_dev(d_st), None if o is None else host(o), None if ob is None else host(ob))
 
 
@@ -48,7 +54,7 @@ def oracle_prefill(cfg, cu, tok, p, st):
                           p["dt_bias"], st["state"], nthreads=NT)
 
 
-def check(cfg, cu, seed, state_std=0.02, conv_std=1.0, extreme=False):
+def check(cfg, cu, seed, state_std=0.02, conv_std=1.0, extreme=False, windows_only=False):
     cu = np.asarray(cu, np.int32)
     n, T = cu.size - 1, int(cu[-1])
     p = inputs.layer_params(cfg, seed)
@@ -57,7 +63,7 @@ def check(cfg, cu, seed, state_std=0.02, conv_std=1.0, extreme=False):
     if extreme:
         p, tok = extreme_params(p), extreme_gates(cfg, tok, seed)
     st = inputs.initial_states(cfg, seed, n, state_std=state_std, conv_std=conv_std)
-    cs, s, o, ob = gpu_prefill(cfg, cu, tok, p, st)
+    cs, s, o, ob = gpu_prefill(cfg, cu, tok, p, st, windows_only=windows_only)
     rcs, rs, ro = oracle_prefill(cfg, cu, tok, p, st)
     np.testing.assert_array_equal(cs, rcs)
     rel = oracle.rel_err(s, rs)
@@ -78,17 +84,20 @@ def test_varlen_with_empty_and_short_sequences():
     check(oracle.make_cfg(), [0, 0, 1, 65, 195, 198, 198, 260], inputs.seed_for(4))
 
 
+@pytest.mark.parametrize("windows_only", [False, True])
 @pytest.mark.parametrize("n", [1100, 4400])
-def test_more_sequences_than_one_plan_pass(n):
+def test_more_sequences_than_one_plan_pass(n, windows_only):
     # The offsets are scanned in passes of 1024 threads, the running maximum and chunk count
     # carried between passes (two and five passes here). Most sequences are empty or a few
-    # tokens long; a few span several chunks around pass boundaries.
+    # tokens long; a few span several chunks around pass boundaries. With windows_only the chunk
+    # table holds them all; without, the plan leaves it to 4400 (more sequences than its list
+    # takes with one head) and takes the sequences of 1100 one by one.
     lens = np.floor(inputs.Gen(inputs.seed_for(4) + n).uniform(0x51, (n,)) * 5).astype(np.int64)
     for b in (1024, 4096):
         if b < n:
             lens[b - 4:b + 3] = [70, 0, 130, 1, 64, 0, 65]
     cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
-    check(oracle.make_cfg(h_k=1, h_v=1), cu, inputs.seed_for(4) + n, state_std=0.0)
+    check(oracle.make_cfg(h_k=1, h_v=1), cu, inputs.seed_for(4) + n, state_std=0.0, windows_only=windows_only)
 
 
 @pytest.mark.parametrize("kw", [
@@ -241,10 +250,12 @@ def test_windows_match_one_window(cu, window):
         np.testing.assert_array_equal(a, b)
 
 
-def test_windows_with_many_sequences():
-    # 600 short sequences, a third of them empty, in windows of two chunks: each window's chain
-    # workgroups walk its chunks across sequence boundaries, in 8 groups cut at sequence starts
-    # (h_v * 8 = 32 strips), resuming states and histories the previous windows left.
+@pytest.mark.parametrize("windows_only", [True, False])
+def test_windows_with_many_sequences(windows_only):
+    # 600 short sequences, a third of them empty, in windows of two chunks. With windows_only each
+    # window's chain workgroups walk its chunks across sequence boundaries, in 8 groups cut at
+    # sequence starts (h_v * 8 = 32 strips), resuming states and histories the previous windows
+    # left; without, every sequence runs in a workgroup of its own and the windows are empty.
     cfg = bx.make_cfg(h_k=2, h_v=4)
     rng = np.random.default_rng(inputs.seed_for(4) + 9)
     lens = rng.integers(1, 100, 600)
@@ -255,8 +266,8 @@ def test_windows_with_many_sequences():
     p = inputs.layer_params(cfg, seed)
     tok = inputs.token_inputs(cfg, seed, T)
     st = inputs.initial_states(cfg, seed, n)
-    full = gpu_prefill(cfg, cu, tok, p, st)
-    win = gpu_prefill(cfg, cu, tok, p, st, window=2)
+    full = gpu_prefill(cfg, cu, tok, p, st, windows_only=windows_only)
+    win = gpu_prefill(cfg, cu, tok, p, st, window=2, windows_only=windows_only)
     for a, b in zip(full, win):
         np.testing.assert_array_equal(a, b)
 

@@ -13,14 +13,16 @@ import pytest
 import baloon_amd as bx
 import oracle
 from oracle import bf16, inputs
-from tests.common import NT, TOL_O_ABS, TOL_STATE_REL, dev, host, state_from_dev, state_to_dev, tabled_chunks
+from tests.common import (NT, TOL_O_ABS, TOL_STATE_REL, dev, extreme_gates, extreme_params, host, state_from_dev,
+                          state_to_dev, tabled_chunks)
 
 pytestmark = pytest.mark.gpu
 
 EDGES = [0, 1, 2, 3, 4, 15, 16, 17, 31, 33, 48, 63, 64, 65, 66, 67, 80, 127, 128, 129, 130]
 
 
-def run(cfg, cu, tok, p, st, gate=None, window=None):
+def run(cfg, cu, tok, p, st, gate=None, window=None, tabled=None, with_o=False):
+    """tabled: how many chunks the plan has to send through the windows. with_o: the gated call writes o too."""
     import torch
     n, T = len(cu) - 1, tok["x"].shape[0]
     size = bx.ix_gdn_prefill_workspace_size if gate is None else bx.ix_gdn_prefill_gated_workspace_size
@@ -35,13 +37,16 @@ def run(cfg, cu, tok, p, st, gate=None, window=None):
     if gate is None:
         assert bx.ix_gdn_prefill(*args, o=o, o_bf16=ob, workspace=ws, workspace_bytes=need) == 0
         torch.cuda.synchronize()
+        assert tabled is None or tabled_chunks(ws, n) == tabled
         return host(d_cs), state_from_dev(d_st), host(o), host(ob)
     y = torch.full((T, cfg.h_v, cfg.d_v), float("nan"), device="cuda")
     yb = torch.zeros(T, cfg.h_v, cfg.d_v, dtype=torch.bfloat16, device="cuda")
     yq = torch.zeros(T * cfg.h_v * cfg.d_v // 32 * 36, dtype=torch.uint8, device="cuda")
-    og = bx.out_gate(dev(gate["z"]), dev(gate["nrm"]), 1e-6, y, yb, yq)
-    assert bx.ix_gdn_prefill_gated(*args, gate=og, workspace=ws, workspace_bytes=need) == 0
+    z, nrm = dev(gate["z"]), dev(gate["nrm"])                  # held: the gate holds addresses alone
+    og = bx.out_gate(z, nrm, 1e-6, y, yb, yq)
+    assert bx.ix_gdn_prefill_gated(*args, o=o if with_o else None, gate=og, workspace=ws, workspace_bytes=need) == 0
     torch.cuda.synchronize()
+    assert tabled is None or tabled_chunks(ws, n) == tabled
     q = torch.zeros_like(yq)
     assert bx.ix_q8_1_quantize(y, q, y.numel()) == 0
     torch.cuda.synchronize()
@@ -59,7 +64,8 @@ def run(cfg, cu, tok, p, st, gate=None, window=None):
 ])
 @pytest.mark.parametrize("longest", [130, 1500])
 def test_many_sequences(kw, n, longest):
-    # longest = 1500: one sequence that the plan leaves to the windows among short ones.
+    # Few heads make the windows cheap: the plan leaves most of these batches' chunks to them, and a
+    # sequence of 1500 tokens in every case. test_by_sequence has the batches it does not.
     cfg = bx.make_cfg(**kw)
     lens = (EDGES * 3)[:n]
     lens[7] = longest
@@ -85,6 +91,106 @@ def test_many_sequences(kw, n, longest):
 
 def chunks(lens):
     return sum((v + 63) // 64 for v in lens)
+
+
+@pytest.mark.parametrize("kw,n", [
+    (dict(h_k=4, h_v=8), 180),                                 # two heads a workgroup
+    (dict(h_k=2, h_v=6, head_map=1, conv_act=1), 220),         # an odd count: the last half repeats a head
+    (dict(h_k=3, h_v=3, conv_act=1), 300),                     # one head a workgroup
+    (dict(h_k=2, h_v=5, d_conv=3, conv_act=1), 260),           # modulo pairing, uneven: 3 and 2 heads
+    (dict(h_k=4, h_v=3, d_conv=2), 300),                       # a q/k head without v heads, one head a workgroup
+    (dict(h_k=3, h_v=6, d_conv=2, conv_act=1), 300),
+    (dict(h_k=4, h_v=8, head_map=1, conv_act=1, q_scale=128 ** -0.5), 180),
+])
+@pytest.mark.parametrize("longest,gates", [(200, "drawn"), (1500, "drawn"), (200, "extreme")])
+def test_by_sequence(kw, n, longest, gates):
+    """Batches whose sequences all run in workgroups of their own, but for one of 1500 tokens (too long a
+    walk beside the others) that the windows take, gated too with and without the caller's o."""
+    cfg = bx.make_cfg(**kw)
+    lens = (EDGES * 15)[:n]
+    lens[7] = longest
+    tabled = chunks([1500]) if longest == 1500 else 0
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, seed = int(cu[-1]), inputs.seed_for(4) + 501 + n + longest
+    p, tok = inputs.layer_params(cfg, seed), inputs.token_inputs(cfg, seed, T)
+    if gates == "extreme":                                     # decays of 0 next to decays of 1 (tests/common.py)
+        p, tok = extreme_params(p), extreme_gates(cfg, tok, seed)
+    st, g = inputs.initial_states(cfg, seed, n), inputs.out_gate_inputs(cfg, seed, T)
+    rcs, rs, ro = oracle.prefill(cfg, cu, tok["x"], st["conv_state"], p["w"], tok["a"], tok["b"], p["A_log"],
+                                 p["dt_bias"], st["state"], nthreads=NT)
+    cs, s, o, ob = run(cfg, cu, tok, p, st, tabled=tabled)
+    np.testing.assert_array_equal(cs, rcs)
+    # Extreme gates: a chunk's cumulative log decay reaches -8,192, where each of the scan's 6 steps rounds
+    # by up to 2^-12; a factor exp(G_t - G_s) takes both ends' errors. (The windows are no closer.)
+    assert oracle.rel_err(s, rs) <= (TOL_STATE_REL if gates == "drawn" else 12 * 2.0 ** -12)
+    assert float(np.max(np.abs(o - ro))) <= TOL_O_ABS
+    np.testing.assert_array_equal(ob, bf16.from_f32(o))
+    gated = run(cfg, cu, tok, p, st, g, tabled=tabled)
+    np.testing.assert_array_equal(gated[0], cs)
+    np.testing.assert_array_equal(gated[1], s)                 # the norm changes no state
+    own = oracle.gated_out(o.astype(np.float64), g["z"], g["nrm"], 1e-6)
+    assert oracle.rel_err(gated[2], own) <= 1e-5               # test_gated_gpu.py's bound on the call's own outputs
+    np.testing.assert_array_equal(gated[3], bf16.from_f32(gated[2]))
+    for kwargs in (dict(with_o=True), dict(window=2)):
+        for u, v in zip(gated, run(cfg, cu, tok, p, st, g, tabled=tabled, **kwargs)):
+            np.testing.assert_array_equal(u, v)
+
+
+@pytest.mark.parametrize("beta_logit", [None, 30.0])
+def test_no_decay_by_sequence(beta_logit):
+    """Decays of 1 (and beta = 1): the blocks of (I + A)^-1 as large as they get, over several chunks."""
+    cfg, n = bx.make_cfg(h_k=4, h_v=8), 100
+    lens = [200 - s % 70 for s in range(n)]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, seed = int(cu[-1]), inputs.seed_for(3) + 43
+    p, tok, st = inputs.layer_params(cfg, seed), dict(inputs.token_inputs(cfg, seed, T)), inputs.initial_states(cfg, seed, n)
+    tok["a"] = bf16.from_f32(np.full(tok["a"].shape, -30.0, np.float32))
+    if beta_logit is not None:
+        tok["b"] = bf16.from_f32(np.full(tok["b"].shape, beta_logit, np.float32))
+    rcs, rs, ro = oracle.prefill(cfg, cu, tok["x"], st["conv_state"], p["w"], tok["a"], tok["b"], p["A_log"],
+                                 p["dt_bias"], st["state"], nthreads=NT)
+    cs, s, o, ob = run(cfg, cu, tok, p, st, tabled=0)
+    np.testing.assert_array_equal(cs, rcs)
+    assert oracle.rel_err(s, rs) <= TOL_STATE_REL
+    assert float(np.max(np.abs(o - ro))) <= TOL_O_ABS
+
+
+@pytest.mark.parametrize("at", ["o", "o_bf16", "z", "y", "y_bf16", None])
+def test_alignment(at):
+    """Outputs and gate inputs off the vector accesses' alignment send the batch through the windows."""
+    import torch
+    cfg, n = bx.make_cfg(h_k=4, h_v=8), 64
+    lens = [1 + s for s in range(n)]
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, seed = int(cu[-1]), inputs.seed_for(4) + 77
+    p, tok, st = inputs.layer_params(cfg, seed), inputs.token_inputs(cfg, seed, T), inputs.initial_states(cfg, seed, n)
+    g = inputs.out_gate_inputs(cfg, seed, T)
+
+    def buf(name, dtype):
+        v = torch.zeros(T * 8 * 128 + 8, dtype=dtype, device="cuda")
+        return v[1 if name == at else 0:][:T * 8 * 128]
+
+    bufs = {name: buf(name, torch.bfloat16 if name in ("o_bf16", "z", "y_bf16") else torch.float32)
+            for name in ("o", "o_bf16", "z", "y", "y_bf16")}
+    bufs["z"].copy_(dev(g["z"]).view(-1))
+    need = bx.ix_gdn_prefill_gated_workspace_size(cfg, n, T)
+    ws, d_st, d_cs = torch.empty(need, dtype=torch.uint8, device="cuda"), state_to_dev(st["state"]), dev(st["conv_state"])
+    nrm = dev(g["nrm"])                                        # held: the gate holds addresses alone
+    og = bx.out_gate(bufs["z"], nrm, 1e-6, bufs["y"], bufs["y_bf16"])
+    assert bx.ix_gdn_prefill_gated(cfg, n, T, dev(cu), dev(tok["x"]), d_cs, dev(p["w"]), dev(tok["a"]), dev(tok["b"]),
+                                   dev(p["A_log"]), dev(p["dt_bias"]), d_st, o=bufs["o"], o_bf16=bufs["o_bf16"], gate=og,
+                                   workspace=ws, workspace_bytes=need) == 0
+    torch.cuda.synchronize()
+    assert tabled_chunks(ws, n) == (0 if at is None else n)
+    rcs, rs, ro = oracle.prefill(cfg, cu, tok["x"], st["conv_state"], p["w"], tok["a"], tok["b"], p["A_log"],
+                                 p["dt_bias"], st["state"], nthreads=NT)
+    o, y = (host(bufs[k]).reshape(T, 8, 128) for k in ("o", "y"))
+    np.testing.assert_array_equal(host(d_cs), rcs)
+    assert oracle.rel_err(state_from_dev(d_st), rs) <= TOL_STATE_REL
+    assert float(np.max(np.abs(o - ro))) <= TOL_O_ABS
+    assert oracle.rel_err(y, oracle.gated_out(o.astype(np.float64), g["z"], g["nrm"], 1e-6)) <= 1e-5
+    np.testing.assert_array_equal(host(bufs["o_bf16"]), bf16.from_f32(o).reshape(-1))
+    np.testing.assert_array_equal(host(bufs["y_bf16"]), bf16.from_f32(y).reshape(-1))
 
 
 @pytest.mark.parametrize("n", [1, 3, 64])
