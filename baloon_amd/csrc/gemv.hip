@@ -230,7 +230,8 @@ mmvq_q8_0_lds_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ 
         xq[(2 * c + 1) * nb + kb] = u32x4{b[5], b[6], b[7], b[8]};
     }
     __syncthreads();
-    for (int row = (int)blockIdx.x * kQLdsWaves + tid / kWave; row < n_out; row += (int)gridDim.x * kQLdsWaves) {
+    // 64 bits: past the last row a wave's next one may lie beyond 2^31.
+    for (long long row = (long long)blockIdx.x * kQLdsWaves + tid / kWave; row < n_out; row += (long long)gridDim.x * kQLdsWaves) {
         const uint8_t* wr = w + (size_t)row * nb * kQ80Bytes;
         float acc[NC];
 #pragma unroll
@@ -299,7 +300,7 @@ void launch_q8_0(const uint8_t* w, const uint8_t* x, float* y, int n_in, int n_o
         hipLaunchKernelGGL(mmvq_q8_0_kernel<NC>, dim3(row_blocks(n_out)), dim3(kGemvThreads), 0, s, w, x, y, n_in, n_out);
         return;
     }
-    const int grid = std::min((n_out + kQLdsWaves - 1) / kQLdsWaves, 2 * device_cu_count(s));
+    const long long grid = std::min((n_out + kQLdsWaves - 1LL) / kQLdsWaves, 2LL * device_cu_count(s));
     hipLaunchKernelGGL(mmvq_q8_0_lds_kernel<NC>, dim3((unsigned)grid), dim3(kQLdsThreads), (unsigned)(NC * kQ81Bytes * nb), s,
                        w, x, y, n_in, n_out);
 }

@@ -31,3 +31,24 @@ def test_q8_0_many_rows(n_in, n_out):
         assert float((np.abs(outs[nc][:nc].astype(np.float64) - ref[:nc]) / sc[:nc]).max()) <= 1e-5
         assert np.isnan(outs[nc][nc:]).all()
         np.testing.assert_array_equal(outs[nc][:nc], outs[8][:nc])
+
+
+def test_q8_0_most_rows():
+    """The largest n_out the call takes (73 GB of one-block rows): the first and last rows hold codes, the others
+    are zero; the row counter of a wave passes 2^31 behind the last one."""
+    import torch
+    n_out = 2 ** 31 - 1
+    if torch.cuda.mem_get_info()[0] < 100e9:
+        pytest.skip("needs 82 GB of device memory")
+    wd, wq = proj.q8_blocks(0x6D4E0A07, 1, 16, 1)
+    xd, xq = proj.q8_blocks(0x6D4E0A07, 5, 1, 1)
+    ref, sc = proj.q8_0_ref(wd, wq, xd, xq)
+    rows, x = dev(proj.pack_q8_0(wd, wq)).view(16, 34), dev(proj.pack_q8_1(xd, xq))
+    w = torch.zeros(n_out * 34, dtype=torch.uint8, device="cuda")
+    w[:8 * 34] = rows[:8].reshape(-1)
+    w[-8 * 34:] = rows[8:].reshape(-1)
+    y = torch.full((n_out + 1,), float("nan"), device="cuda")
+    assert bx.ix_mmvq_q8_0(w, x, y, 32, n_out, 1) == 0
+    got = host(torch.cat([y[:8], y[n_out - 8:n_out]]))
+    assert float((np.abs(got.astype(np.float64) - ref[0]) / sc[0]).max()) <= 1e-5
+    assert bool(torch.isnan(y[n_out])) and int(torch.count_nonzero(y[8:n_out - 8])) == 0
