@@ -1401,21 +1401,29 @@ __global__ void __launch_bounds__(256) out_gate_kernel(const float* __restrict__
     out_gate_head(g, row, o[row + lane], o[row + lane + kWave], lane);
 }
 
-// The same norm over one window's chunks, a wave per row in a grid of at most kGateBlocks workgroups:
-// from the window buffer (64 rows per chunk) for the gated prefill without a caller o, else from o.
-constexpr unsigned kGateBlocks = 4096;
+// The same norm over one window's chunks: grid (chunks, parts of a chunk's rows), each workgroup its 4
+// waves over a part, kGateRows rows of a full chunk per wave. From the window buffer (64 rows per chunk)
+// for the gated prefill without a caller o, else from o. One row after the other over a grid of 4,096
+// workgroups (a 64-bit division per row) made gated calls slower: 4096 tokens 221 us, four prompts of 1000 234,
+// with one row per wave 211 and 221, two 205 and 220, four 208 and 223. Where the plan may have left the windows
+// nothing the grid stays at 4,096 workgroups, so that an empty one costs little, and they stride over the chunks.
+constexpr int kGateRows = 2;
 __global__ void __launch_bounds__(256) out_gate_window_kernel(const PrefillParams p, const OutGate g) {
     const int lane = threadIdx.x & (kWave - 1);
-    const long long per = (long long)kChunk * p.L.h_v, rows = per * p.W;       // h_v rows per token
-    for (long long r = (long long)blockIdx.x * 4 + threadIdx.x / kWave; r < rows; r += (long long)gridDim.x * 4) {
-        const int lc = (int)(r / per), in = (int)(r % per);
-        ChunkGeo c;
-        if (!chunk_geo(p, p.cb + lc, c)) return;
-        if (in >= c.len * p.L.h_v) continue;
-        const size_t row = ((size_t)c.t0 * p.L.h_v + in) * kD;
-        const float* o = p.o + (p.o_win ? (size_t)r * kD : row);
-        out_gate_head(g, row, o[lane], o[lane + kWave], lane);
+    ChunkGeo c;
+    for (int lc = (int)blockIdx.x; lc < p.W && chunk_geo(p, p.cb + lc, c); lc += (int)gridDim.x) {
+        const int rows = c.len * p.L.h_v;                                      // h_v rows per token
+        const size_t row0 = (size_t)c.t0 * p.L.h_v;
+        const float* o = p.o + (p.o_win ? (size_t)lc * kChunk * p.L.h_v : row0) * kD;
+        for (int r = (int)blockIdx.y * 4 + threadIdx.x / kWave; r < rows; r += (int)gridDim.y * 4) {
+            const float* q = o + (size_t)r * kD;
+            out_gate_head(g, (row0 + r) * kD, q[lane], q[lane + kWave], lane);
+        }
     }
+}
+inline dim3 gate_grid(const PrefillParams& p) {
+    const int parts = std::min((kChunk / 4 * p.L.h_v + kGateRows - 1) / kGateRows, 65535);
+    return dim3((unsigned)(p.by_seq ? std::min(p.W, std::max(4096 / parts, 1)) : p.W), (unsigned)parts);
 }
 
 }  // namespace
@@ -1577,9 +1585,7 @@ static hipError_t prefill_impl(const ix_gdn_cfg* cfg, int n_seq, int total_T, co
             default: launch_prefill<4>(p, tgrid, cgrid, cblock, silu, s); break;
         }
         if (gwin || (gate && p.by_seq))
-            hipLaunchKernelGGL(out_gate_window_kernel,
-                               dim3((unsigned)std::min<long long>(((long long)p.W * kChunk * cfg->h_v + 3) / 4, kGateBlocks)),
-                               dim3(256), 0, s, p, og);
+            hipLaunchKernelGGL(out_gate_window_kernel, gate_grid(p), dim3(256), 0, s, p, og);
     }
     if (gate && !gwin && !p.by_seq)
         hipLaunchKernelGGL(out_gate_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, p.o, og, rows);
