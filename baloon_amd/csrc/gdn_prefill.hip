@@ -1584,11 +1584,15 @@ static hipError_t prefill_impl(const ix_gdn_cfg* cfg, int n_seq, int total_T, co
             case 3: launch_prefill<3>(p, tgrid, cgrid, cblock, silu, s); break;
             default: launch_prefill<4>(p, tgrid, cgrid, cblock, silu, s); break;
         }
-        if (gwin || (gate && p.by_seq))
-            hipLaunchKernelGGL(out_gate_window_kernel, gate_grid(p), dim3(256), 0, s, p, og);
+        if (gwin) hipLaunchKernelGGL(out_gate_window_kernel, gate_grid(p), dim3(256), 0, s, p, og);
     }
-    if (gate && !gwin && !p.by_seq)
+    if (gate && !gwin && p.by_seq) {                           // every chunk of the table
+        p.cb = 0;
+        p.W = p.NC;
+        hipLaunchKernelGGL(out_gate_window_kernel, gate_grid(p), dim3(256), 0, s, p, og);
+    } else if (gate && !gwin) {
         hipLaunchKernelGGL(out_gate_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, p.o, og, rows);
+    }
     return hipGetLastError();
 }
 
