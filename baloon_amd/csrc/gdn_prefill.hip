@@ -1494,6 +1494,7 @@ static bool by_sequence(const ixg::PrefillParams& p, const ixg::OutGate& g, bool
     auto on = [](const void* q, uintptr_t a) { return (reinterpret_cast<uintptr_t>(q) & (a - 1)) == 0; };
     if (p.single || p.L.C >= 1 << 22 || p.n_seq > ixg::kTriFragBytes / 4 * p.L.h_v) return false;
     if (!on(p.o_win ? nullptr : p.o, 16) || !on(p.o_bf16, 8)) return false;
+    if (p.n_seq * ixg::seq_workgroups(p.L) * ixg::kSeqThreads > 0xffffffffLL) return false;   // a launch's threads
     if (gated && !(on(g.z, 8) && on(g.nrm, 16) && on(g.y, 16) && on(g.y_bf16, 8) && on(g.y_q8_1, 4))) return false;
     return p.n_seq * ixg::seq_workgroups(p.L) >= kSeqWorkgroups;
 }

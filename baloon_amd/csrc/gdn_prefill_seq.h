@@ -4,7 +4,9 @@
 
 namespace ixg {
 
-// Workgroups per sequence.
+constexpr int kSeqThreads = 512;
+
+// Workgroups (of kSeqThreads) per sequence.
 long long seq_workgroups(const Layer& L);
 
 // Prefill of every sequence of the batch that has no chunk in the plan's chunk table: states, outputs

@@ -38,7 +38,6 @@
 namespace ixg {
 namespace {
 
-constexpr int kSeqThreads = 512;
 constexpr int kSeqWaves = kSeqThreads / kWave;
 // LDS (bytes): key planes; query planes, then A and the waves' v inputs in the same place; per head
 // M, the diagonal blocks of T, and G, beta, exp(G), exp(G_last - G); the outputs, 64 rows of 128

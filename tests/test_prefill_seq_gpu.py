@@ -262,3 +262,24 @@ def test_plan_routes(n, gated, tabled):
         assert bx.ix_gdn_prefill(*args, o_bf16=yb, workspace=ws, workspace_bytes=need) == 0
     torch.cuda.synchronize()
     assert tabled_chunks(ws, n) == (chunks(lens) if tabled else 0)
+
+
+def test_more_workgroups_than_a_launch_takes():
+    """2,048 sequences with 4,096 q/k heads would be 2^32 threads by sequence: they stay in the windows. (One v
+    head, so that the states fit; inputs of one token each, of which k and q are zero.)"""
+    import torch
+    if torch.cuda.mem_get_info()[0] < 60e9:
+        pytest.skip("needs 40 GB of device memory")
+    cfg, n = bx.make_cfg(h_k=4096, h_v=1), 2048
+    C, bf = cfg.channels, dict(dtype=torch.bfloat16, device="cuda")
+    x = torch.zeros(n, C, **bf)
+    x[:, -128:] = 1.0
+    a, cs, zero = torch.zeros(n, 1, **bf), torch.zeros(n, C, 3, **bf), torch.zeros(1, device="cuda")
+    need = bx.ix_gdn_prefill_window_workspace_size(cfg, n, n, 16, False)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    assert bx.ix_gdn_prefill(cfg, n, n, torch.arange(n + 1, dtype=torch.int32, device="cuda"), x, cs, torch.zeros(C, 4, **bf),
+                             a, a, zero, zero, torch.zeros(n, 1, 128, 128, device="cuda"), workspace=ws,
+                             workspace_bytes=need) == 0
+    torch.cuda.synchronize()
+    assert tabled_chunks(ws, n) == n
+    assert bool((cs[:, -128:, 2] == 1).all())
