@@ -9,7 +9,8 @@ error behaviour -- every call returns a ``hipError_t`` code (0 = success), with
 PyTorch is only plumbing here: tensors supply device memory and the current stream. Every
 tensor argument must live on the GPU; the functions pass raw device pointers to the C ABI.
 There is no CPU fallback: if the library is missing, :func:`lib` raises. The launchers' arguments
-are converted by the extension ``_bind`` (csrc/bind.cpp); the other symbols are bound with ctypes.
+are converted by the extension ``_bind`` (csrc/bind.cpp), or by ctypes where it does not take them;
+the other symbols are bound with ctypes.
 """
 from __future__ import annotations
 
@@ -76,6 +77,42 @@ def make_cfg(h_k=16, h_v=32, d_k=128, d_v=128, d_conv=4, head_map=HEAD_MOD, conv
     return Cfg(h_k, h_v, d_k, d_v, d_conv, head_map, conv_act, q_scale, l2_eps)
 
 
+# Arguments of every symbol: a layer description (c) or output gate (g) by reference, a tensor's address (p), the
+# stream (s); i, l, z and f are an int, a long long, a size_t and a float.
+_TYPES = {**dict.fromkeys("cgps", ctypes.c_void_p), "i": ctypes.c_int, "l": ctypes.c_longlong, "z": ctypes.c_size_t,
+          "f": ctypes.c_float}
+_I, _Z = ctypes.c_int, ctypes.c_size_t
+_SIGNATURES = {
+    "ix_gdn_step": ("pppppppiiis", _I),
+    "ix_gdn_conv_step": ("ppppiis", _I),
+    "ix_gdn_l2_norm": ("piifs", _I),
+    "ix_gdn_beta_gate": ("pis", _I),
+    "ix_gdn_out_norm": ("ppppiifs", _I),
+    "ix_gdn_channels": ("c", _I),
+    "ix_gdn_decode_workspace_size": ("ci", _Z),
+    "ix_gdn_decode": ("cippppppppppps", _I),
+    "ix_gdn_prefill_workspace_size": ("cii", _Z),
+    "ix_gdn_prefill": ("ciippppppppppppzs", _I),
+    "ix_gdn_decode_gated": ("cippppppppppgps", _I),
+    "ix_gdn_prefill_gated_workspace_size": ("cii", _Z),
+    "ix_gdn_prefill_window_workspace_size": ("ciiii", _Z),
+    "ix_gdn_prefill_gated": ("ciipppppppppppgpzs", _I),
+    "ix_gdn_window_record_size": ("cii", _Z),
+    "ix_gdn_decode_window": ("ciippppppppppps", _I),
+    "ix_gdn_decode_window_mfma": ("ciippppppppppps", _I),
+    "ix_gdn_commit_window": ("ciippppps", _I),
+    "ix_bf16_gemv": ("ppplls", _I),
+    "ix_bf16_gemv_pair": ("ppplpplls", _I),
+    "ix_bf16_gemv_split": ("pppllis", _I),
+    "ix_mmvq_q8_0": ("pppiiis", _I),
+    "ix_gdn_in_proj_width": ("c", _I),
+    "ix_gdn_in_proj": ("ciippppppps", _I),
+    "ix_gdn_version": ("", ctypes.c_char_p),
+    "ix_gdn_decode_noalloc": ("cipppppppppps", _I),
+    "ix_q8_1_quantize": ("ppls", _I),
+    "ix_gdn_commit_window_layers": ("ciiippppps", _I),
+}
+
 _lib = None
 
 
@@ -87,42 +124,10 @@ def lib() -> ctypes.CDLL:
     if not os.path.exists(LIB_PATH):
         raise RuntimeError(f"{LIB_PATH} is missing: build it with `python -m baloon_amd.build`")
     L = ctypes.CDLL(LIB_PATH)
-    P, I, F, Z, LL = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_size_t, ctypes.c_longlong
-    sig = {
-        "ix_gdn_step": ([P, P, P, P, P, P, P, I, I, I, P], I),
-        "ix_gdn_conv_step": ([P, P, P, P, I, I, P], I),
-        "ix_gdn_l2_norm": ([P, I, I, F, P], I),
-        "ix_gdn_beta_gate": ([P, I, P], I),
-        "ix_gdn_out_norm": ([P, P, P, P, I, I, F, P], I),
-        "ix_gdn_channels": ([P], I),
-        "ix_gdn_decode_workspace_size": ([P, I], Z),
-        "ix_gdn_decode": ([P, I, P, P, P, P, P, P, P, P, P, P, P, P], I),
-        "ix_gdn_prefill_workspace_size": ([P, I, I], Z),
-        "ix_gdn_prefill": ([P, I, I, P, P, P, P, P, P, P, P, P, P, P, P, Z, P], I),
-        "ix_gdn_decode_gated": ([P, I, P, P, P, P, P, P, P, P, P, P, P, P, P], I),
-        "ix_gdn_prefill_gated_workspace_size": ([P, I, I], Z),
-        "ix_gdn_prefill_window_workspace_size": ([P, I, I, I, I], Z),
-        "ix_gdn_prefill_gated": ([P, I, I, P, P, P, P, P, P, P, P, P, P, P, P, P, Z, P], I),
-        "ix_gdn_window_record_size": ([P, I, I], Z),
-        "ix_gdn_decode_window": ([P, I, I, P, P, P, P, P, P, P, P, P, P, P, P], I),
-        "ix_gdn_decode_window_mfma": ([P, I, I, P, P, P, P, P, P, P, P, P, P, P, P], I),
-        "ix_gdn_commit_window": ([P, I, I, P, P, P, P, P, P], I),
-        "ix_bf16_gemv": ([P, P, P, LL, LL, P], I),
-        "ix_bf16_gemv_pair": ([P, P, P, LL, P, P, LL, LL, P], I),
-        "ix_bf16_gemv_split": ([P, P, P, LL, LL, I, P], I),
-        "ix_mmvq_q8_0": ([P, P, P, I, I, I, P], I),
-        "ix_gdn_in_proj_width": ([P], I),
-        "ix_gdn_in_proj": ([P, I, I, P, P, P, P, P, P, P, P], I),
-        "ix_gdn_version": ([], ctypes.c_char_p),
-        "ix_gdn_decode_noalloc": ([P, I, P, P, P, P, P, P, P, P, P, P, P], I),
-        "ix_q8_1_quantize": ([P, P, LL, P], I),
-        "ix_gdn_commit_window_layers": ([P, I, I, I, P, P, P, P, P, P], I),
-    }
-    for name, (args, res) in sig.items():
+    for name, (args, res) in _SIGNATURES.items():
         fn = getattr(L, name)
-        fn.argtypes = args
+        fn.argtypes = [_TYPES[t] for t in args]
         fn.restype = res
-        _bind.bind(name, ctypes.cast(fn, P).value)
     _lib = L
     return L
 
@@ -145,32 +150,56 @@ def _stream(s) -> int | None:
     return getattr(s, "cuda_stream", s)
 
 
-class _Unbuilt:
-    """Stands for the extension until it has been built."""
+class _ArgumentError(ctypes.ArgumentError, TypeError):
+    """An argument that fits no C type: ctypes' own error, and a TypeError like those of the extension."""
+
+
+def _byref(v, least):
+    if v is not None and ctypes.sizeof(v) < ctypes.sizeof(least):
+        raise TypeError("structure too small")
+    return ctypes.byref(v)
+
+
+def _through_ctypes(name, args) -> int:
+    """A launcher's call with ctypes' conversions: for arguments that the extension leaves to it (anything but
+    plain tensors, ints, floats, structures and streams)."""
+    convert = {"c": lambda v: _byref(v, Cfg), "g": lambda v: None if v is None else _byref(v, OutGate),
+               "p": _ptr, "s": _stream}
+    fn = getattr(lib(), name)
+    args = [convert[t](v) if t in convert else v for t, v in zip(_SIGNATURES[name][0], args)]
+    try:
+        return fn(*args)
+    except ctypes.ArgumentError as e:
+        raise _ArgumentError(*e.args) from None
+
+
+class _NoExtension:
+    """Stands for the extension until the first call."""
 
     def __getattr__(self, name):
         return getattr(_import_bind(), name)
 
 
 def _import_bind():
+    """Load the extension and hand it the library's addresses."""
     global _bind
     import importlib
 
+    L = lib()
     import torch  # noqa: F401  (before _bind, which uses its libraries)
     try:
         m = importlib.import_module("._bind", __name__)
-        m.setup(lib, _ptr, ctypes.Structure.__mro__[-2])      # the base of every ctypes type
-    except (ImportError, TypeError) as e:                      # TypeError: built from older sources
+        m.setup(_through_ctypes, ctypes.Structure.__mro__[-2])    # the base of every ctypes type
+    except (ImportError, TypeError) as e:                          # TypeError: built from older sources
         raise RuntimeError(f"{PKG}/_bind.so is missing or does not load: build it with "
                            "`python -m baloon_amd.build`") from e
+    for name in _SIGNATURES:
+        m.bind(name, ctypes.cast(getattr(L, name), ctypes.c_void_p).value)
     _bind = m
     return m
 
 
-try:
-    _import_bind()
-except RuntimeError:
-    _bind = _Unbuilt()
+_bind = _NoExtension()
 
 
 def check(name: str, code: int) -> None:

@@ -6,11 +6,11 @@
 // torch.cuda, a conversion object per argument): one token through the five drop-in launchers took
 // 38 us for 16 us of kernels. Here an argument is read from the tensor's C++ object.
 //
-// Arguments are converted by the C parameter's type: pointers from tensors (on the GPU, contiguous)
-// or None, descriptions from ctypes structures, the stream from None (torch's current one), a
-// torch stream or an address. Anything but a plain torch.Tensor or Parameter goes through the
-// mirror's own _ptr, which refuses or reads it as before. The library's functions are found by
-// the mirror (lib()), which hands their addresses over.
+// Arguments are converted by the C parameter's type: pointers from tensors (plain torch.Tensor or
+// Parameter, on the GPU, contiguous) or None, descriptions from ctypes structures, numbers from ints and
+// floats, the stream from None (torch's current one), a torch stream or an address. A call with any other argument
+// goes as a whole to the mirror's ctypes path, which reads or refuses it. The mirror hands over the addresses
+// of the library's functions.
 #include <Python.h>
 
 #include <cstring>
@@ -19,112 +19,125 @@
 
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/device_lazy_init.h>
 
 #include "ix_gdn.h"
 
 namespace {
 
-PyObject* g_load = nullptr;     // lib(): loads the library and binds the addresses below
-PyObject* g_ptr = nullptr;      // _ptr()
+PyObject* g_other = nullptr;    // the mirror's ctypes path: (name, arguments) -> code
 PyObject* g_cdata = nullptr;    // the base of every ctypes type
 
-// Every converter returns with a Python error set if the argument does not fit.
-void* tensor_ptr(PyObject* o) {
+// The converters set `other` for an argument that they leave to ctypes.
+void* tensor_ptr(PyObject* o, bool& other) {
     if (o == Py_None) return nullptr;
     if (THPVariable_CheckExact(o)) {
         const at::Tensor& t = THPVariable_Unpack(o);
         if (t.is_cuda() && t.layout() == c10::kStrided && t.is_contiguous()) return t.data_ptr();
     }
-    PyObject* r = PyObject_CallOneArg(g_ptr, o);             // other objects, and the refusals
-    if (!r) return nullptr;
-    void* p = r == Py_None ? nullptr : PyLong_AsVoidPtr(r);
-    Py_DECREF(r);
-    return p;
+    other = true;
+    return nullptr;
 }
 
-long long integer(PyObject* o) {
-    PyObject* i = PyNumber_Index(o);
-    if (!i) return 0;
-    const unsigned long long v = PyLong_AsUnsignedLongLongMask(i);
-    Py_DECREF(i);
-    return (long long)v;
+long long integer(PyObject* o, bool& other) {
+    if (PyLong_Check(o)) return (long long)PyLong_AsUnsignedLongLongMask(o);
+    other = true;
+    return 0;
 }
 
-// Any ctypes instance of the C structure's size or more (a program may declare its own mirror of it).
+float real(PyObject* o, bool& other) {
+    if (PyFloat_Check(o)) return (float)PyFloat_AS_DOUBLE(o);
+    other = true;
+    return 0.0f;
+}
+
+// Any ctypes instance of the C structure's size or more (a program may declare its own mirror of it). The
+// caller holds it.
 template <class T>
-const T* structure(PyObject* o) {
-    const int is = PyObject_IsInstance(o, g_cdata);
-    if (is < 0) return nullptr;
+const T* structure(PyObject* o, bool& other) {
     Py_buffer b;
-    if (!is) {
-        PyErr_Format(PyExc_TypeError, "expected a ctypes instance, got %R", (PyObject*)Py_TYPE(o));
-        return nullptr;
+    if (PyObject_IsInstance(o, g_cdata) == 1 && PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) == 0) {
+        const T* p = b.len >= (Py_ssize_t)sizeof(T) ? static_cast<const T*>(b.buf) : nullptr;
+        PyBuffer_Release(&b);
+        if (p) return p;
     }
-    if (PyObject_GetBuffer(o, &b, PyBUF_SIMPLE) != 0) return nullptr;
-    const T* p = b.len >= (Py_ssize_t)sizeof(T) ? static_cast<const T*>(b.buf) : nullptr;
-    PyBuffer_Release(&b);                                    // the caller holds the structure
-    if (!p) PyErr_SetString(PyExc_TypeError, "structure too small");
-    return p;
+    PyErr_Clear();
+    other = true;
+    return nullptr;
 }
 
-hipStream_t stream(PyObject* o) {
-    if (o == Py_None) return c10::hip::getCurrentHIPStream().stream();
-    if (PyLong_Check(o)) return static_cast<hipStream_t>(PyLong_AsVoidPtr(o));
-    PyObject* v = PyObject_GetAttrString(o, "cuda_stream");
-    if (!v) {                                                // a ctypes.c_void_p
-        PyErr_Clear();
-        v = PyObject_GetAttrString(o, "value");
-        if (!v) return nullptr;
-        if (v == Py_None) {
+hipStream_t stream(PyObject* o, bool& other) {
+    if (o == Py_None) {
+        other = torch::utils::is_device_in_bad_fork(at::kCUDA);   // torch.cuda refuses such a process
+        return other ? nullptr : c10::hip::getCurrentHIPStream().stream();
+    }
+    PyObject* v = PyLong_Check(o) ? Py_NewRef(o) : PyObject_GetAttrString(o, "cuda_stream");
+    if (v && PyLong_Check(v)) {
+        void* p = PyLong_AsVoidPtr(v);
+        if (!PyErr_Occurred()) {
             Py_DECREF(v);
-            return nullptr;
+            return static_cast<hipStream_t>(p);
         }
     }
-    hipStream_t s = static_cast<hipStream_t>(PyLong_AsVoidPtr(v));
-    Py_DECREF(v);
-    return s;
+    Py_XDECREF(v);
+    PyErr_Clear();
+    other = true;
+    return nullptr;
 }
 
 template <class T>
 struct Arg {                                                 // pointers to device memory
-    static T of(PyObject* o) { return static_cast<T>(tensor_ptr(o)); }
+    static T of(PyObject* o, bool& other) { return static_cast<T>(tensor_ptr(o, other)); }
 };
 template <>
 struct Arg<const ix_gdn_cfg*> {
-    static const ix_gdn_cfg* of(PyObject* o) { return structure<ix_gdn_cfg>(o); }
+    static const ix_gdn_cfg* of(PyObject* o, bool& other) { return structure<ix_gdn_cfg>(o, other); }
 };
 template <>
 struct Arg<const ix_gdn_out_gate*> {
-    static const ix_gdn_out_gate* of(PyObject* o) {
-        return o == Py_None ? nullptr : structure<ix_gdn_out_gate>(o);
+    static const ix_gdn_out_gate* of(PyObject* o, bool& other) {
+        return o == Py_None ? nullptr : structure<ix_gdn_out_gate>(o, other);
     }
 };
 template <>
 struct Arg<int> {
-    static int of(PyObject* o) { return (int)integer(o); }
+    static int of(PyObject* o, bool& other) { return (int)integer(o, other); }
 };
 template <>
 struct Arg<long long> {
-    static long long of(PyObject* o) { return integer(o); }
+    static long long of(PyObject* o, bool& other) { return integer(o, other); }
 };
 template <>
 struct Arg<size_t> {
-    static size_t of(PyObject* o) { return (size_t)integer(o); }
+    static size_t of(PyObject* o, bool& other) { return (size_t)integer(o, other); }
 };
 template <>
 struct Arg<float> {
-    static float of(PyObject* o) { return (float)PyFloat_AsDouble(o); }
+    static float of(PyObject* o, bool& other) { return real(o, other); }
 };
 template <>
 struct Arg<hipStream_t> {
-    static hipStream_t of(PyObject* o) { return stream(o); }
+    static hipStream_t of(PyObject* o, bool& other) { return stream(o, other); }
 };
 
+PyObject* through_ctypes(const char* name, PyObject* const* args, Py_ssize_t n) {
+    PyObject* t = PyTuple_New(n);
+    if (!t) return nullptr;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        Py_INCREF(args[i]);
+        PyTuple_SET_ITEM(t, i, args[i]);
+    }
+    PyObject* r = PyObject_CallFunction(g_other, "sO", name, t);
+    Py_DECREF(t);
+    return r;
+}
+
 template <class... A, size_t... I>
-PyObject* invoke(hipError_t (*fn)(A...), PyObject* const* args, std::index_sequence<I...>) {
-    // Braces: converted from left to right, up to the first error.
-    const std::tuple<A...> v{(PyErr_Occurred() ? A{} : Arg<A>::of(args[I]))...};
-    if (PyErr_Occurred()) return nullptr;
+PyObject* invoke(hipError_t (*fn)(A...), const char* name, PyObject* const* args, std::index_sequence<I...>) {
+    bool other = false;
+    // Braces: converted from left to right, up to the first that is left to ctypes.
+    const std::tuple<A...> v{(other ? A{} : Arg<A>::of(args[I], other))...};
+    if (other) return through_ctypes(name, args, (Py_ssize_t)sizeof...(A));
     hipError_t e;
     Py_BEGIN_ALLOW_THREADS
     e = fn(std::get<I>(v)...);
@@ -133,22 +146,17 @@ PyObject* invoke(hipError_t (*fn)(A...), PyObject* const* args, std::index_seque
 }
 
 template <class... A>
-PyObject* call(hipError_t (*&fn)(A...), const char* name, PyObject* const* args, Py_ssize_t n) {
+PyObject* call(hipError_t (*fn)(A...), const char* name, PyObject* const* args, Py_ssize_t n) {
     if (n != (Py_ssize_t)sizeof...(A)) {
         PyErr_Format(PyExc_TypeError, "%s takes %d arguments, got %d", name, (int)sizeof...(A), (int)n);
         return nullptr;
     }
+    if (!fn) {
+        PyErr_Format(PyExc_RuntimeError, "%s is not bound", name);
+        return nullptr;
+    }
     try {
-        if (!fn) {
-            PyObject* r = PyObject_CallNoArgs(g_load);
-            if (!r) return nullptr;
-            Py_DECREF(r);
-            if (!fn) {
-                PyErr_Format(PyExc_RuntimeError, "%s is not bound", name);
-                return nullptr;
-            }
-        }
-        return invoke(fn, args, std::index_sequence_for<A...>{});
+        return invoke(fn, name, args, std::index_sequence_for<A...>{});
     } catch (const std::exception& e) {                      // from torch's accessors
         if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
         return nullptr;
@@ -181,12 +189,12 @@ PyObject* bind(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
-// setup(lib, _ptr, ctypes' base type)
+// setup(the ctypes path, ctypes' base type)
 PyObject* setup(PyObject*, PyObject* args) {
-    PyObject *l, *p, *c;
-    if (!PyArg_ParseTuple(args, "OOO", &l, &p, &c)) return nullptr;
-    Py_INCREF(l); Py_INCREF(p); Py_INCREF(c);
-    g_load = l; g_ptr = p; g_cdata = c;
+    PyObject *o, *c;
+    if (!PyArg_ParseTuple(args, "OO", &o, &c)) return nullptr;
+    Py_INCREF(o); Py_INCREF(c);
+    g_other = o; g_cdata = c;
     Py_RETURN_NONE;
 }
 

@@ -1,7 +1,8 @@
-"""The Python mirror's argument conversion (csrc/bind.cpp): what it refuses before any launch, on
-the CPU, and on the GPU the streams and tensors it accepts."""
+"""The Python mirror's argument conversion (csrc/bind.cpp, and ctypes for what that leaves to it): what it
+takes and refuses before any launch, on the CPU, and on the GPU the streams and tensors it accepts."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
@@ -42,20 +43,39 @@ def test_descriptions_of_other_types():
         bx.ix_gdn_decode(ctypes.c_int(1), 1, *args, s=0)
 
 
+class Stream:
+    def __init__(self, cuda_stream):
+        self.cuda_stream = cuda_stream
+
+
+def test_arguments_left_to_ctypes():
+    """What ctypes converts is taken as ctypes takes it, and what it refuses is its ArgumentError."""
+    for ints in ((0, 1), (ctypes.c_int(0), ctypes.c_int(1)), (np.int64(0), np.int32(1)), (False, 1), (2 ** 40, 1)):   # no rows
+        for eps in (1e-6, 1, ctypes.c_float(1e-6), np.float32(1e-6)):
+            for s in (0, Stream(0), Stream(None), ctypes.c_void_p(0), ctypes.c_void_p(), 2 ** 64, -1):
+                assert bx.ix_gdn_l2_norm(None, *ints, eps, s) == bx.HIP_ERROR_INVALID_VALUE
+    assert bx.ix_bf16_gemv(None, None, None, ctypes.c_longlong(0), 0, 0) == bx.HIP_ERROR_INVALID_VALUE
+    for args in ((4.5, 1, 1e-6, 0), (4, "a", 1e-6, 0), (4, 1, "a", 0), (4, 1, 10 ** 400, 0), (4, 1, 1e-6, np.int64(0)),
+                 (4, 1, 1e-6, 0.0), (ctypes.c_longlong(4), ctypes.c_float(1), 1e-6, 0)):
+        with pytest.raises(ctypes.ArgumentError):
+            bx.ix_gdn_l2_norm(None, *args)
+
+
 @pytest.mark.gpu
 def test_streams_and_tensors():
     x = torch.randn(6, 128, device="cuda")
     want = x / torch.sqrt((x.double() ** 2).sum(1, keepdim=True) + 1e-6).float()
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
-    for how in ("current", "object", "address"):
+    for how in ("current", "object", "address", "c_void_p"):
         y = torch.nn.Parameter(x.clone(), requires_grad=False)
         side.wait_stream(torch.cuda.current_stream())
         if how == "current":
             with torch.cuda.stream(side):
                 assert bx.ix_gdn_l2_norm(y, 6, 128, 1e-6) == 0
         else:
-            assert bx.ix_gdn_l2_norm(y, 6, 128, 1e-6, side if how == "object" else side.cuda_stream) == 0
+            s = side if how == "object" else side.cuda_stream
+            assert bx.ix_gdn_l2_norm(y, 6, 128, 1e-6, ctypes.c_void_p(s) if how == "c_void_p" else s) == 0
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         assert float((y - want).abs().max()) <= 1e-6
