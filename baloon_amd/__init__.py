@@ -9,8 +9,8 @@ error behaviour -- every call returns a ``hipError_t`` code (0 = success), with
 PyTorch is only plumbing here: tensors supply device memory and the current stream. Every
 tensor argument must live on the GPU; the functions pass raw device pointers to the C ABI.
 There is no CPU fallback: if the library is missing, :func:`lib` raises. The launchers' arguments
-are converted by the extension ``_bind`` (csrc/bind.cpp), or by ctypes where it does not take them;
-the other symbols are bound with ctypes.
+are converted by the extension ``_bind`` (csrc/bind.cpp), or by ctypes where it does not take them or is
+missing; the other symbols are bound with ctypes.
 """
 from __future__ import annotations
 
@@ -162,7 +162,7 @@ def _byref(v, least):
 
 def _through_ctypes(name, args) -> int:
     """A launcher's call with ctypes' conversions: for arguments that the extension leaves to it (anything but
-    plain tensors, ints, floats, structures and streams)."""
+    plain tensors, ints, floats, structures and streams), and for every call where there is no extension."""
     convert = {"c": lambda v: _byref(v, Cfg), "g": lambda v: None if v is None else _byref(v, OutGate),
                "p": _ptr, "s": _stream}
     fn = getattr(lib(), name)
@@ -180,19 +180,29 @@ class _NoExtension:
         return getattr(_import_bind(), name)
 
 
+class _Ctypes:
+    """Stands for the extension where it is missing or does not load."""
+
+    def __getattr__(self, name):
+        return lambda *args: _through_ctypes(name, args)
+
+
 def _import_bind():
     """Load the extension and hand it the library's addresses."""
     global _bind
     import importlib
 
     L = lib()
-    import torch  # noqa: F401  (before _bind, which uses its libraries)
     try:
+        import torch  # noqa: F401  (before _bind, which uses its libraries)
         m = importlib.import_module("._bind", __name__)
         m.setup(_through_ctypes, ctypes.Structure.__mro__[-2])    # the base of every ctypes type
     except (ImportError, TypeError) as e:                          # TypeError: built from older sources
-        raise RuntimeError(f"{PKG}/_bind.so is missing or does not load: build it with "
-                           "`python -m baloon_amd.build`") from e
+        import warnings
+        warnings.warn(f"{PKG}/_bind.so is missing or does not load ({e}): calls go through ctypes, some 3 us slower "
+                      "each. Build it with `python -m baloon_amd.build`", RuntimeWarning, stacklevel=3)
+        _bind = _Ctypes()
+        return _bind
     for name in _SIGNATURES:
         m.bind(name, ctypes.cast(getattr(L, name), ctypes.c_void_p).value)
     _bind = m

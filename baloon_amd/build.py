@@ -1,6 +1,7 @@
 """Build libixgdn.so (HIP, gfx950) in-tree with hipcc, and _bind.so, the Python mirror's call path.
 
     python -m baloon_amd.build           # compile every csrc/*.hip and link the library; csrc/bind.cpp
+    python baloon_amd/build.py           # the same without importing the package (and, without torch, no _bind.so)
 
 Each translation unit is compiled for gfx950 only, with packed-FP32 instruction selection
 disabled (-packed-fp32-ops), and with kernel resource-usage remarks captured to
@@ -81,8 +82,12 @@ def _build_bind() -> None:
     """_bind.so: host C++ against the Python and torch headers (csrc/bind.cpp)."""
     import sysconfig
 
-    import torch
-    from torch.utils.cpp_extension import include_paths
+    try:
+        import torch
+        from torch.utils.cpp_extension import include_paths
+    except ImportError as e:                     # C and C++ callers need the library alone
+        print(f"no Python binding: {e}")
+        return
 
     rocm = os.path.dirname(os.path.dirname(HIPCC))
     libs = os.path.join(os.path.dirname(torch.__file__), "lib")
@@ -104,7 +109,6 @@ def build(verbose: bool = False) -> str:
     with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
         bind = ex.submit(_build_bind)
         results = list(ex.map(_compile, srcs))
-        bind.result()
     objs = [o for o, _ in results]
     remarks = "".join(r for _, r in results)
     with open(RESOURCE_REPORT, "w") as f:
@@ -115,6 +119,7 @@ def build(verbose: bool = False) -> str:
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stderr}")
     os.replace(tmp, LIB)
+    bind.result()                                # the library stands without it
     if verbose:
         print(open(RESOURCE_REPORT).read(), end="")
         print(f"built {LIB}")

@@ -1,12 +1,16 @@
 """The Python mirror's argument conversion (csrc/bind.cpp, and ctypes for what that leaves to it): what it
 takes and refuses before any launch, on the CPU, and on the GPU the streams and tensors it accepts."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 import torch
 
 import baloon_amd as bx
+from baloon_amd import build
 
 
 def test_refusals():
@@ -59,6 +63,48 @@ def test_arguments_left_to_ctypes():
                  (4, 1, 1e-6, 0.0), (ctypes.c_longlong(4), ctypes.c_float(1), 1e-6, 0)):
         with pytest.raises(ctypes.ArgumentError):
             bx.ix_gdn_l2_norm(None, *args)
+
+
+def test_library_without_the_extension():
+    """Where _bind.so does not load, the library's symbols are there, and the calls go through ctypes, with a
+    warning."""
+    code = """
+import sys, warnings
+sys.modules["baloon_amd._bind"] = None
+import baloon_amd as bx
+assert bx.version().startswith("ixgdn") and bx.ix_gdn_in_proj_width(bx.make_cfg()) > 0
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    for _ in range(2):
+        assert bx.ix_gdn_beta_gate(None, 4, 0) == bx.HIP_ERROR_INVALID_VALUE
+assert len(seen) == 1 and "_bind.so" in str(seen[0].message), seen
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300,
+                   cwd=os.path.dirname(os.path.dirname(os.path.abspath(bx.__file__))))
+
+
+@pytest.mark.parametrize("torch_there", [False, True])
+def test_library_is_linked_without_the_extension(monkeypatch, tmp_path, torch_there):
+    """Without torch the library alone is built; where the extension's build fails, the library is linked first."""
+    for name in ("BUILD", "LIB", "BIND", "RESOURCE_REPORT"):
+        monkeypatch.setattr(build, name, str(tmp_path / name))
+    if not torch_there:
+        monkeypatch.setitem(sys.modules, "torch", None)
+    monkeypatch.setattr(build, "_compile", lambda src: (src + ".o", ""))
+
+    def run(cmd, **_):
+        if "-ltorch_python" in cmd:
+            return subprocess.CompletedProcess(cmd, 1, "", "refused")
+        open(cmd[cmd.index("-o") + 1], "w").close()
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    monkeypatch.setattr(build.subprocess, "run", run)
+    if torch_there:
+        with pytest.raises(RuntimeError, match="refused"):
+            build.build()
+    else:
+        build.build()
+    assert os.path.exists(build.LIB) and not os.path.exists(build.BIND)
 
 
 @pytest.mark.gpu
