@@ -1492,8 +1492,9 @@ static void launch_prefill(const ixg::PrefillParams& p, dim3 tgrid, dim3 cgrid, 
 // Which of the sequences then do is decided on the device, from their lengths (plan_kernel): with
 // SiLU and output gate, U[1, 2048] tokens, 16 q/k and 32 v heads, 12 sequences take 643 us in windows (741 by
 // sequence), 14 742 us by sequence (757 in windows), 16 753 (877), 32 847 (1,744); plain ones 426 (506), 497 in
-// windows (510), 516 (572), 580 (1,131).
-constexpr long long kSeqWorkgroups = 176;
+// windows (510), 516 (572), 580 (1,131). Below 14 (224 workgroups) the plan nearly always chose the windows,
+// and choosing takes 8 us (its own passes and two launches that find nothing): 11 sequences of U[1, 755] 166 -> 173.
+constexpr long long kSeqWorkgroups = 224;
 static bool by_sequence(const ixg::PrefillParams& p, const ixg::OutGate& g, bool gated) {
     auto on = [](const void* q, uintptr_t a) { return (reinterpret_cast<uintptr_t>(q) & (a - 1)) == 0; };
     if (p.single || p.L.C >= 1 << 22 || p.n_seq > ixg::kTriFragBytes / 4 * p.L.h_v) return false;
