@@ -322,7 +322,7 @@ void launch_tiles(const InProj& p, int cols, hipStream_t s) {
 // the same: the launch for the remaining columns), as measured for 100 to 4096 rows, N = 3,088 to
 // 12,352 and K = 1024 to 2048: 0.048 per 64 x 64 tile (4096 rows, N = 12,352: 513 us); two 128 x 128 tiles per CU in
 // 39, one in 26 (512 rows: 50 us against 70; 2048 rows: 128); a 256 x 256 tile per CU in 58 (4096 rows:
-// 196 us, 1,055 TFLOP/s, against 242 with 128 x 128).
+// 202 to 207 us with the launch for the remaining columns, 1,000 to 1,023 TFLOP/s, against 242 with 128 x 128).
 int tile_columns(const InProj& p, hipStream_t s) {
     auto on16 = [](const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     if (p.y || !on16(p.x) || !on16(p.z)) return 0;

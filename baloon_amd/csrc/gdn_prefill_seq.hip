@@ -12,27 +12,29 @@
 // waves, and every A operand read from LDS serves all its tiles. Per chunk, with S the state at
 // its start and the notation of gdn_prefill.hip, in four phases that end at a barrier:
 //   1. conv, activation and L2 norm of the q rows (waves 0-3) and k rows (waves 4-7) into
-//      split-bf16 planes; the heads' decay scans;
-//   2. the 10 + 10 lower-triangle blocks of K K^T and Q K^T, shared out over the waves, with the
-//      heads' decays (A, M); the 16 x 16 diagonal blocks of T = (I + A)^-1 by substitution in fp32
-//      (waves 6 and 7); W = K S and Q S of the wave's columns; the previous chunk's outputs leave
-//      LDS, a row per half wave (whole 512-byte lines; the gated norm of a row sits in one half
-//      wave);
-//   3. A over the query planes; V (conv of the wave's v channels) and X = diag(beta) (V - diag(Gam) W);
-//   4. D by block forward substitution on X (D_i = T_ii (X_i - sum_{j<i} A_ij D_j); the blocks of
-//      T below the diagonal are never formed), O = diag(Gam) Q S + M D into LDS, S' = gam S +
-//      K^T diag(E) D.
+//      split-bf16 planes; the heads' decay scans (waves 0 and 5, or wave 0);
+//   2. waves 0-3: the 10 + 10 lower-triangle blocks of K K^T and Q K^T in six tasks (block_row), with
+//      the heads' decays (A, M); the four 16 x 16 diagonal blocks of T = (I + A)^-1 by substitution in fp32,
+//      each in the wave whose task formed it (tasks 1, 3, 4, 5: waves 1, 3, 0 and 2). All waves: W = K S
+//      and Q S of their columns. Waves 4-7: the previous chunk's outputs leave LDS, a row per half wave
+//      (whole 512-byte lines; the gated norm of a row sits in one half wave);
+//   3. into the query planes' space: A's blocks of rows 2 and 3 left of the diagonal blocks' 32 columns
+//      (waves 0 and 2), T_10 and T_32 (waves 3 and 1); V (conv of the wave's v channels) and X =
+//      diag(beta) (V - diag(Gam) W);
+//   4. D in two steps of 32 rows, D_b = [T_00 0; T_10 T_11] X_b of the step's diagonal block, the second on
+//      X less the A blocks' product with the first (the blocks of T left of those are never formed);
+//      O = diag(Gam) Q S + M D into LDS; S' = gam S + K^T diag(E) D.
 // Products are split-bf16 MFMA as in gdn_prefill.hip, accumulator tiles feeding the next product
 // as B operands (kperm order).
 //
-// What bounds it: vector instructions and the latency of the dependent phases. A chunk of two heads
-// takes ~42,000 cycles on a CU (phases 1 to 4: 7.7, 18.5, 3.1 and 12 thousand); of these its two
-// waves per SIMD issue vector work for ~22,000 (two transcendentals for every activation and
-// gate) and matrix work for ~13,000. Workgroups of one head with 16 columns a wave, two per CU,
-// repeat the q/k work for each head and spill: 967 us for 32 sequences of U[1, 2048] tokens (16 q/k,
-// 32 v heads, gated) against 700. Products and vector work share a phase where waves w and w + 4
-// (one SIMD) can take them in opposite order; operands of the long product loops are read one
-// step ahead. The whole batch, against windows of chunk kernel and chain: 716 us, 1,732 before.
+// What bounds it: vector instructions and the latency of the dependent phases. With SiLU and output gate
+// a chunk of two heads takes 52,800 cycles on a CU (phases 1 to 4: 10.6, 23.7, 7.6 and 10.9 thousand; plain
+// 6.3, 15.1, 3.5 and 11.1, in all 36,000); it issues 36,400 vector and matrix instructions of a wave, 9,100 on each
+// SIMD at 4 cycles or more, and keeps a SIMD's matrix unit busy for 12,800 cycles. Workgroups of one
+// head with 16 columns a wave, two per CU, repeat the q/k work for each head and spill: 967 us against 700
+// (an earlier form, 32 sequences of U[1, 2048] tokens, 16 q/k, 32 v heads, gated). Products and vector
+// work share a phase where waves w and w + 4 (one SIMD) can take them in opposite order; operands of the
+// long product loops are read one step ahead. That batch with SiLU: 845-857 us, in windows 1,744.
 #include "gdn_prefill_seq.h"
 
 namespace ixg {
@@ -397,7 +399,7 @@ __global__ void __launch_bounds__(kSeqThreads) seq_kernel(const SeqArgs args) {
             phase();
             // 2. blocks of K K^T and Q K^T, transposed (lane (li, lg4) holds t = 16 br + li, s = 16 bc +
             // 4 lg4 + r), with each head's decays: M split into its fragments, the diagonal blocks of
-            // A (waves 1, 3, 4, 5) in fp32 and inverted, the others held until the query planes are free
+            // A (tasks 1, 3, 4, 5) in fp32 and inverted, the others held until the query planes are free
             if (w < 4) {
 #pragma clang loop unroll(disable)
                 for (int task = w; task < 6; task = task < 4 && !(w & 1) ? 4 + (w >> 1) : 6) {

@@ -186,7 +186,11 @@ size_t ix_gdn_prefill_window_workspace_size(const ix_gdn_cfg* cfg, int n_seq, in
  *   workspace: 256-byte aligned device memory of at least
  *   ix_gdn_prefill_window_workspace_size(cfg, n_seq, total_T, 1, 0) bytes (windows of one
  *   chunk); the prefill uses windows of as many chunks as the workspace holds, e.g.
- *   ix_gdn_prefill_workspace_size() bytes. */
+ *   ix_gdn_prefill_workspace_size() bytes.
+ * In batches of many sequences the shorter ones may run in a workgroup each instead of in windows, as the
+ * number of sequences, heads and lengths and the outputs' alignment (o 16, o_bf16 8 bytes) make
+ * it worth while. Both agree to the rounding of the split-bf16 products (about 1e-5), so the low bits of a
+ * sequence's results may depend on the batch it is in; they do not depend on the workspace. */
 hipError_t ix_gdn_prefill(const ix_gdn_cfg* cfg, int n_seq, int total_T, const int32_t* cu_seqlens,
                           const uint16_t* x, uint16_t* conv_state, const uint16_t* conv_w, const uint16_t* a,
                           const uint16_t* b, const float* A_log, const float* dt_bias, float* state, float* o,
@@ -201,7 +205,7 @@ size_t ix_gdn_prefill_gated_workspace_size(const ix_gdn_cfg* cfg, int n_seq, int
 /* ix_gdn_prefill followed by the gated output norm of every (token, v head) row:
  * gate->z, gate->y, gate->y_bf16 are [total_T][h_v][d_v]; workspace_bytes must be at least
  * ix_gdn_prefill_window_workspace_size(cfg, n_seq, total_T, 1, 1) (windows of one chunk;
- * ix_gdn_prefill_gated_workspace_size() gives the default windows). */
+ * ix_gdn_prefill_gated_workspace_size() gives the default windows). gate->y_bf16 may be gate->z itself. */
 hipError_t ix_gdn_prefill_gated(const ix_gdn_cfg* cfg, int n_seq, int total_T, const int32_t* cu_seqlens,
                                 const uint16_t* x, uint16_t* conv_state, const uint16_t* conv_w,
                                 const uint16_t* a, const uint16_t* b, const float* A_log, const float* dt_bias,
