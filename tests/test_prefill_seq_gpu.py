@@ -284,3 +284,41 @@ def test_more_workgroups_than_a_launch_takes():
     torch.cuda.synchronize()
     assert tabled_chunks(ws, n) == n
     assert bool((cs[:, -128:, 2] == 1).all())
+
+
+def test_graph_replays():
+    """A captured call (the plan, walks, windows and the norm over the table's chunks) replays like eager calls,
+    each from the states the one before left, with eager work in between."""
+    import torch
+    cfg, lens = bx.make_cfg(h_k=4, h_v=8, conv_act=1), [1500] + [1 + (53 * s) % 190 for s in range(120)]
+    n, T = len(lens), sum(lens)
+    seed = inputs.seed_for(4) + 91
+    p, tok, st = inputs.layer_params(cfg, seed), inputs.token_inputs(cfg, seed, T), inputs.initial_states(cfg, seed, n)
+    g = inputs.out_gate_inputs(cfg, seed, T)
+    cu = dev(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+    x, a, b, w, A, dt, z, nrm = (dev(v) for v in (tok["x"], tok["a"], tok["b"], p["w"], p["A_log"], p["dt_bias"], g["z"], g["nrm"]))
+    need = bx.ix_gdn_prefill_gated_workspace_size(cfg, n, T)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+
+    def buffers():
+        return (dev(st["conv_state"]), state_to_dev(st["state"]), torch.zeros(T, 8, 128, device="cuda"),
+                torch.zeros(T, 8, 128, device="cuda"))
+
+    def call(cs, state, o, y):
+        assert bx.ix_gdn_prefill_gated(cfg, n, T, cu, x, cs, w, a, b, A, dt, state, o=o, gate=bx.out_gate(z, nrm, 1e-6, y),
+                                       workspace=ws, workspace_bytes=need) == 0
+
+    eager, graphed = buffers(), buffers()
+    call(*buffers())                                           # outside the capture once
+    torch.cuda.synchronize()
+    assert tabled_chunks(ws, n) == chunks([1500])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(*graphed)
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        call(*eager)
+        torch.cuda.synchronize()
+        for u, v in zip(graphed, eager):
+            np.testing.assert_array_equal(host(u), host(v))
